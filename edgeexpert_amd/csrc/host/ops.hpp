@@ -26,6 +26,18 @@ constexpr uint32_t kProjMaxK = 8192;       // longest reduction (gemm.hpp kProjM
 constexpr uint32_t kUnitThreads = 256;          // grouped MoE units (moe_prefill.hpp)
 constexpr uint32_t kUnitStride = 128 + 8;       // halves per LDS activation row of a unit
 constexpr uint32_t kGroupMaxTiles = 8192 / 128 + 256;  // tiles the device planner takes (moe_prefill.hpp)
+// int8 rows over a block of tokens (gemm_q8.hpp)
+constexpr uint32_t kQ8RowTokens = 4;            // most tokens that run the decode kernels once per token
+constexpr uint32_t kQ8FewTokens = 64;           // most tokens on the K-split form (down at 96 tokens: 12.4 against
+                                                // 14.7 us for the tile, gate/up 18.6 against 19.6; at 192 30 against
+                                                // 14.8 and 32 against 20)
+constexpr uint32_t kQ8BlockThreads = 512;       // threads of the K-split form
+constexpr uint32_t kQ8TileThreads = 256;        // threads, tokens and weight rows of the tile
+constexpr uint32_t kQ8TileTok = 64;
+constexpr uint32_t kQ8TileRows = 64;
+constexpr uint32_t q8_tile_lds_bytes(uint32_t k) {
+    return 2u * (kQ8TileTok * 128u + kQ8TileRows * 64u) + 4u * kQ8TileRows * (k / 64u);
+}
 // the pipelined tile of the prefill GEMM (gemm.hpp proj_pl_lds_bytes)
 constexpr uint32_t proj_pl_lds_bytes(uint32_t k) { return 3u * kProjBM * 72u * 2u + 4u * kProjBN * (k / 64u); }
 static_assert(proj_pl_lds_bytes(kProjMaxK) <= 160u * 1024u, "pipelined tile exceeds the LDS of a CU");
@@ -632,7 +644,12 @@ private:
 // S/Kernels/MoE/SharedExpertInt8.swift:55-210: the fused int8 gate/up/act
 // (shared_int8_gate_up_act_simd; gate and up kept in fp32 up to the
 // activation) and the int8 down GEMV. tokens > 1 runs the same for a block
-// of inputs x + t·x_stride into y + t·y_stride, act_scratch [tokens][f].
+// of inputs x + t·x_stride into y + t·y_stride, act_scratch [tokens][f]: up to
+// kQ8RowTokens tokens, and rows of x that are not 16-byte aligned, as the
+// decode kernels once per token (each row the decode form's bits), else on the
+// matrix cores (gemm_q8.hpp: the same factored fp32 sums in another order;
+// 13.7 against 53 us for 16 tokens at 2816 x 2112, 62 against 1463 for 512; at
+// 4 tokens 11.1 against 17.4, left to the rows for their bits).
 class SharedExpertInt8 {
 public:
     explicit SharedExpertInt8(const Module& m) : m_(m), gemv_(m) {}
@@ -656,6 +673,15 @@ public:
         Q8Mat g = {static_cast<const uint8_t*>(gate.weights), gate.scales, gate.biases};
         Q8Mat u = {static_cast<const uint8_t*>(up.weights), up.scales, up.biases};
         NormArg na = stage;
+        // a block of tokens on the matrix cores (gemm_q8.hpp)
+        if (tokens > kQ8RowTokens && na.mode == kStageCopy && aligned(x, 16) && x_stride % 8 == 0 &&
+            aligned(act_scratch, 16)) {
+            const Q8Mat dn = {static_cast<const uint8_t*>(down.weights), down.scales, down.biases};
+            if (!aligned(dn.w, 16)) return fail(TFQ_E_INVAL, "weights are not 16-byte aligned");
+            int rc = launch_block(stream, g, u, true, x, act_scratch, tokens, f, d, x_stride, f);
+            if (rc) return rc;
+            return launch_block(stream, dn, dn, false, act_scratch, y, tokens, d, f, f, y_stride);
+        }
         const SegShape sh = seg_shape(d / 16, 4);
         char name[64];
         // 16-byte aligned rows of x in the copy mode: the form whose staging is
@@ -677,6 +703,27 @@ public:
     }
 
 private:
+    // n int8 rows of k codes over `tokens` inputs: few tokens as row tiles
+    // with K split over a block's wavefronts, more as 64 x 64 tiles
+    int launch_block(void* stream, const Q8Mat& a, const Q8Mat& b, bool gated, const uint16_t* x, uint16_t* y,
+                     uint32_t tokens, uint32_t n, uint32_t k, uint32_t ldx, uint32_t ldy) const {
+        const bool tile = tokens > kQ8FewTokens;
+        const uint32_t nt = tokens <= 16 ? 1 : tokens <= 32 ? 2 : 4;        // 16-token tiles per block
+        const uint32_t rows = tile ? (gated ? kQ8TileRows / 2 : kQ8TileRows) : 16, toks = tile ? kQ8TileTok : 16 * nt;
+        char name[64];
+        if (tile) std::snprintf(name, sizeof(name), "tfq_q8_tile%s", gated ? "_gated" : "");
+        else std::snprintf(name, sizeof(name), "tfq_q8_block_%s_t%u", gated ? "gated_r2" : "r1", nt);
+        hipFunction_t fn = m_.get(name);
+        if (!fn) return fail(TFQ_E_NOT_LOADED, "kernel %s is not in the code object", name);
+        void* gated_args[] = {(void*)&a, (void*)&b, &x, &y, &tokens, &n, &k, &ldx, &ldy};
+        void* plain_args[] = {(void*)&a, &x, &y, &tokens, &n, &k, &ldx, &ldy};
+        return hip_check(hipModuleLaunchKernel(fn, (n + rows - 1) / rows, (tokens + toks - 1) / toks, 1,
+                                               tile ? kQ8TileThreads : kQ8BlockThreads, 1, 1,
+                                               tile ? q8_tile_lds_bytes(k) : 0, (hipStream_t)stream,
+                                               gated ? gated_args : plain_args, nullptr),
+                         name);
+    }
+
     const Module& m_;
     DequantInt8GEMV gemv_;
 };
@@ -810,9 +857,9 @@ private:
 
 // S/Kernels/Prefill/MoE/PrefillSharedExpert.swift:4-60 (encodeBlock): the
 // shared expert over `tokens` rows x + t·x_stride -> y + t·y_stride. The
-// reference runs the decode form once per row; here int8 weights run the
-// decode kernels with a token dimension (one launch each for gate/up/act and
-// down), and int4 weights run the prefill GEMM (gate, up -> fp16 in the
+// reference runs the decode form once per row; here int8 weights run
+// SharedExpertInt8's block form (one launch each for gate/up/act and down),
+// and int4 weights run the prefill GEMM (gate, up -> fp16 in the
 // workspace, gelu_mul_fp16 as in SharedExpertInt4's GPU sequence, then
 // down), whose kernel choice by token count picks the weight stream for few
 // tokens.

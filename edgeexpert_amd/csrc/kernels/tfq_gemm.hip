@@ -1,6 +1,8 @@
 // tfq_gemm.hip — the prefill dequant-fused GEMM: the 64-token MFMA projection tile
-// and the few-token weight stream, int4 and 3-bit, fp16 and bf16 activations.
+// and the few-token weight stream, int4 and 3-bit, fp16 and bf16 activations; the
+// int8 rows over a block of tokens (shared expert).
 #include "entry_points.hpp"
+#include "gemm_q8.hpp"
 
 #define TFQ_GEMM(TAG, BITS, DT, X_BF16)                                                          \
     extern "C" __global__ __launch_bounds__(kProjGemmThreads) void tfq_gemm_##TAG##_##DT(        \
@@ -36,3 +38,34 @@ TFQ_SKINNY_C(q3, 3, f16, false, 1)
 TFQ_SKINNY_C(q3, 3, f16, false, 2)
 TFQ_SKINNY_C(q3, 3, bf16, true, 1)
 TFQ_SKINNY_C(q3, 3, bf16, true, 2)
+
+// int8 rows over a block of tokens (gemm_q8.hpp): RT row tiles, NTT token tiles per block.
+#define TFQ_Q8_BLOCK(RT, NTT)                                                                    \
+    extern "C" __global__ __launch_bounds__(kQ8BlockThreads, 2) void tfq_q8_block_r##RT##_t##NTT(  \
+        Q8Mat m, const uint16_t* X, uint16_t* Y, uint32_t M, uint32_t N, uint32_t K,             \
+        uint32_t ldx, uint32_t ldy) {                                                            \
+        gemm_q8_block<RT, NTT, false>(m, m, X, Y, M, N, K, ldx, ldy);                            \
+    }
+#define TFQ_Q8_BLOCK_GATED(RT, NTT)                                                              \
+    extern "C" __global__ __launch_bounds__(kQ8BlockThreads, 2) void                             \
+        tfq_q8_block_gated_r##RT##_t##NTT(Q8Mat gate, Q8Mat up, const uint16_t* X, uint16_t* Y,  \
+                                          uint32_t M, uint32_t N, uint32_t K, uint32_t ldx,      \
+                                          uint32_t ldy) {                                        \
+        gemm_q8_block<RT, NTT, true>(gate, up, X, Y, M, N, K, ldx, ldy);                         \
+    }
+TFQ_Q8_BLOCK(1, 1) TFQ_Q8_BLOCK(1, 2) TFQ_Q8_BLOCK(1, 4)
+TFQ_Q8_BLOCK_GATED(2, 1) TFQ_Q8_BLOCK_GATED(2, 2) TFQ_Q8_BLOCK_GATED(2, 4)
+// many tokens: 64 tokens x 64 rows per block. Two wavefronts per SIMD asked
+// for, so that 256 registers are the bound and the accumulators, which the
+// scaling reads, stay in vector registers.
+extern "C" __global__ __launch_bounds__(kQ8TileThreads, 2) void tfq_q8_tile(Q8Mat m, const uint16_t* X, uint16_t* Y,
+                                                                         uint32_t M, uint32_t N, uint32_t K,
+                                                                         uint32_t ldx, uint32_t ldy) {
+    gemm_q8_tile<false>(m, m, X, Y, M, N, K, ldx, ldy);
+}
+extern "C" __global__ __launch_bounds__(kQ8TileThreads, 2) void tfq_q8_tile_gated(Q8Mat gate, Q8Mat up,
+                                                                               const uint16_t* X, uint16_t* Y,
+                                                                               uint32_t M, uint32_t N, uint32_t K,
+                                                                               uint32_t ldx, uint32_t ldy) {
+    gemm_q8_tile<true>(gate, up, X, Y, M, N, K, ldx, ldy);
+}

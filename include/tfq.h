@@ -505,8 +505,11 @@ size_t tfq_prefill_shared_expert_workspace_bytes(uint32_t weight_bits, uint32_t 
 
 /* The shared expert over a block of `tokens` rows: y + t*y_stride =
  * shared(x + t*x_stride) for t < tokens (strides in halves). int8 weights
- * run the decode kernels over all rows in one launch each, so each row is
- * bit-identical to tfq_shared_expert_q8. int4 weights run the prefill GEMM:
+ * run up to 4 tokens (and rows of x that are not 16-byte aligned) on the
+ * decode kernels, each row bit-identical to tfq_shared_expert_q8, and more
+ * tokens on the matrix cores with the same factored sums (exact products of
+ * code and activation, fp32 accumulation, fp32 scale and bias) in another
+ * order. int4 weights run the prefill GEMM:
  * gate and up are stored to the workspace in fp16 before gelu_mul (the
  * rounding of the reference's GPU sequence, SharedExpertInt4.swift:30-94),
  * then down; tfq_shared_expert_q4 keeps gate/up in fp32 instead, so the two

@@ -165,6 +165,46 @@ def test_prefill_shared_expert_config4_shape(ctx, stream, bits, rows):
         assert rel < TOL, f"row {r}: rel={rel}"
 
 
+@pytest.mark.parametrize("rows,d,f", [(5, 128, 64), (16, 192, 4096), (17, 4096, 320), (32, 2816, 704), (33, 64, 128),
+                                      (64, 320, 192), (65, 704, 2112), (130, 192, 64), (70, 64, 4096)])
+def test_prefill_shared_expert_int8_matrix_cores(ctx, stream, rows, d, f):
+    # from 5 tokens on the int8 block runs on the matrix cores: 16-token tiles
+    # with K split over eight wavefronts (up to 64 tokens; K from fewer groups
+    # than wavefronts to 64), then 64 x 64 tiles (K of 1, 3, 5, 11, 33 and 64
+    # groups); d and f leave partial row tiles, rows partial token tiles
+    print(f"[pshared8] rows={rows} d={d} f={f}", flush=True)
+    mats = _synthetic(6, f"pshared8m/{d}x{f}", d, f, 8)
+    x, got = _prefill_case(ctx, stream, 8, rows, d, f, d + 8, d + 3, mats, 14)
+    for r in sorted({0, 1, 15, 16, 31, 63, 64, rows // 2, rows - 2, rows - 1} & set(range(rows))):
+        ref = oracle.shared_expert_int8(*mats, from_f16_bits(x[r, :d]), d, f)
+        rel = oracle.rel_error(got[r], ref)
+        assert rel < TOL, f"row {r}: rel={rel}"
+
+
+@pytest.mark.parametrize("rows", [6, 66])
+def test_prefill_shared_expert_int8_keeps_rows_apart(ctx, stream, rows):
+    # an infinity in one row makes that row NaN (as inf * 0 codes and inf - inf
+    # do in the decode form) and leaves every other row's bits as they were
+    d, f = 256, 128
+    mats = _synthetic(8, "pshared8inf", d, f, 8)
+    outs = []
+    for bad in (False, True):
+        x = synth.f16_vector(15, f"pshared8inf/x{rows}", rows * d).reshape(rows, d).copy()
+        if bad:
+            x[rows // 2, 7] = 0x7C00
+        y = _dev(np.full(rows * d, SENTINEL, np.uint16))
+        n = ops.prefill_shared_expert_workspace_bytes(8, rows, f)
+        gate, up, down = mats
+        ops.PrefillSharedExpert(ctx, weight_bits=8).encode_block(
+            stream, _dev(x), y, _proj(gate, f, d), _proj(up, f, d), _proj(down, d, f), DeviceBuffer(n), n, rows, d, f,
+            d, d)
+        stream.sync()
+        outs.append(y.download(np.uint16, rows * d).reshape(rows, d))
+    others = [r for r in range(rows) if r != rows // 2]
+    assert np.array_equal(outs[0][others], outs[1][others])
+    assert np.all(np.isnan(from_f16_bits(outs[1][rows // 2])))
+
+
 def test_prefill_shared_expert_rejects_bad_contract(ctx, stream):
     b = _dev(np.zeros(1 << 16, np.uint8))
     p = ops.Q4Projection(b, b, b, rows=64, cols=128)
