@@ -38,6 +38,13 @@ constexpr uint32_t kQ8TileRows = 64;
 constexpr uint32_t q8_tile_lds_bytes(uint32_t k) {
     return 2u * (kQ8TileTok * 128u + kQ8TileRows * 64u) + 4u * kQ8TileRows * (k / 64u);
 }
+// router logits of a block of tokens on the matrix cores: from these many
+// tokens and (token, expert) pairs on. Its time hardly depends on the tokens
+// (128 experts x 2816: 8.8 us for 96 tokens, 9.3 for 512), the per-token form's
+// does (9.0 and 36.4; 40 experts x 1088: 5.4 against 10.8 us at 512 and 5.2
+// against 4.4 at 128).
+constexpr uint32_t kRouterBlockTokens = 96;
+constexpr uint32_t kRouterBlockRows = 96 * 128;
 // the pipelined tile of the prefill GEMM (gemm.hpp proj_pl_lds_bytes)
 constexpr uint32_t proj_pl_lds_bytes(uint32_t k) { return 3u * kProjBM * 72u * 2u + 4u * kProjBN * (k / 64u); }
 static_assert(proj_pl_lds_bytes(kProjMaxK) <= 160u * 1024u, "pipelined tile exceeds the LDS of a CU");
@@ -929,15 +936,25 @@ public:
         if (!r.weights || !r.scales || !r.biases || !hidden || !out_idx || !out_w || !logits)
             return fail(TFQ_E_INVAL, "null pointer argument");
         if (!aligned(r.weights, 16)) return fail(TFQ_E_INVAL, "weights are not 16-byte aligned");
-        const SegShape sh = seg_shape(d / 16, 4);
         char name[64];
-        std::snprintf(name, sizeof(name), "tfq_prefill_router_logits_s%u_p%u", sh.seg, sh.p);
-        const uint32_t rows_per_block = (kBlock / 64) * (64 / sh.seg);
-        const uint32_t gx = (r.num_experts + rows_per_block - 1) / rows_per_block;
         uint32_t E = r.num_experts;
-        void* args[] = {(void*)&r.weights, (void*)&r.scales, (void*)&r.biases, &hidden, &stride,
-                        (void*)&r.effective_scale, &logits, &E, &d};
-        int rc = launch2(m_, name, gx, T, kBlock, d * 6, stream, args);
+        int rc;
+        if (T >= kRouterBlockTokens && (uint64_t)T * E >= kRouterBlockRows && aligned(hidden, 16) && stride % 8 == 0 &&
+            aligned(r.effective_scale, 16)) {
+            // 16 tokens x 16 experts per block on the matrix cores (gemm_q8.hpp)
+            std::snprintf(name, sizeof(name), "tfq_router_block_c%u", (d + 511) / 512);
+            Q8Mat m = {r.weights, r.scales, r.biases};
+            void* args[] = {&m, &hidden, &stride, (void*)&r.effective_scale, &logits, &T, &E, &d};
+            rc = launch2(m_, name, (E + 15) / 16, (T + 15) / 16, kQ8BlockThreads, 0, stream, args);
+        } else {
+            const SegShape sh = seg_shape(d / 16, 4);
+            std::snprintf(name, sizeof(name), "tfq_prefill_router_logits_s%u_p%u", sh.seg, sh.p);
+            const uint32_t rows_per_block = (kBlock / 64) * (64 / sh.seg);
+            const uint32_t gx = (E + rows_per_block - 1) / rows_per_block;
+            void* args[] = {(void*)&r.weights, (void*)&r.scales, (void*)&r.biases, &hidden, &stride,
+                            (void*)&r.effective_scale, &logits, &E, &d};
+            rc = launch2(m_, name, gx, T, kBlock, d * 6, stream, args);
+        }
         if (rc) return rc;
         void* sargs[] = {&logits, (void*)&r.per_expert_scale, &out_idx, &out_w, &out_wf, &E, &top_k};
         return launch2(m_, "tfq_prefill_select", T, 1, 256, 0, stream, sargs);

@@ -42,9 +42,10 @@ constexpr int kQ8RedTokens = 2;                           // token tiles per LDS
 constexpr int q8_round(int NTT) { return NTT < kQ8RedTokens ? NTT : kQ8RedTokens; }
 
 // 8 byte codes (two words, element order) as exact fp16 values: each pair of
-// bytes into the mantissas of two halves of exponent 2^10, minus 1024.
-__device__ __forceinline__ h8 q8_to_h8(uint32_t w0, uint32_t w1) {
-    const h2 m = {(_Float16)1024.0f, (_Float16)1024.0f};
+// bytes into the mantissas of two halves of exponent 2^10, minus base (1024
+// for the codes 0..255 themselves).
+__device__ __forceinline__ h8 q8_to_h8(uint32_t w0, uint32_t w1, _Float16 base = (_Float16)1024.0f) {
+    const h2 m = {base, base};
     const h2 p[4] = {__builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, w0, 0x04010400u)) - m,
                      __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, w0, 0x04030402u)) - m,
                      __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, w1, 0x04010400u)) - m,
@@ -369,6 +370,153 @@ __device__ __forceinline__ void gemm_q8_tile(const Q8Mat& m0, const Q8Mat& m1, c
             if (n < N && t < M) Y[(size_t)t * ldy + n] = f2h(acc[r]);
         }
     }
+}
+
+// ------------------------------------------------ router, many tokens ----
+
+// Logits of a block of prompt tokens: logits[t][e] = Σ_g s·Σ q·x + b·Σ x over
+// x = h[t] ⊙ eff, as router_logits (gemv.hpp) forms them, in another order of
+// the fp32 sums. The product of two fp16 values has 22 significant bits, so
+// x·2^k = hi + lo with two fp16 values, exactly (k scales the largest |x| of
+// the wavefront's slice of the token to [2^14, 2^15): nothing overflows, and
+// what lo loses to fp16's smallest step lies 2^38 below that largest value);
+// both go through the matrix cores with exact products. A slice that holds an
+// infinity takes k = -17, which keeps every finite x finite, and lo = 0 beside
+// a non-finite hi: sums come out infinite or NaN where the scalar form's do.
+//
+// 512 tokens, 128 experts x 2816: 36.4 us once per token (fp32 VALU dots over
+// the whole router for every token), 9.3 us here; relative error against 64
+// bits 2.0e-7 and 1.15e-7.
+//
+// Block: 8 wavefronts, 16 experts x 16 tokens, wave w the groups CNT·w ..
+// (CNT = ceil(K / 512), all loaded before the first use; groups past K take
+// x = 0). Operand layout as in gemm_q8_block.
+template <int CNT>
+__device__ __forceinline__ void router_block(const Q8Mat& m, const uint16_t* __restrict__ h, uint32_t stride,
+                                             const uint16_t* __restrict__ eff, float* __restrict__ logits, uint32_t T,
+                                             uint32_t E, uint32_t K) {
+    __shared__ f32x4 red[kQ8BlockWaves][64];
+    __shared__ __attribute__((aligned(16))) uint32_t sb[16 * (kQ8MaxK / 64)];
+    __shared__ __attribute__((aligned(16))) float inv[kQ8BlockWaves][16];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t r16 = lane & 15u, q = lane >> 4;
+    const uint32_t G = K >> 6, n0 = blockIdx.x * 16u, t0 = blockIdx.y * 16u, g0 = wave * CNT;
+    const uint32_t row = n0 + r16 < E ? n0 + r16 : E - 1;               // experts past E: clamped, not stored
+    const uint32_t t = t0 + r16 < T ? t0 + r16 : T - 1;                 // tokens past T: clamped, not stored
+    const uint32_t piece = (q >> 1) | ((q & 1u) << 1);                  // as in gemm_q8_block
+    const uint8_t* wrow = m.w + (size_t)row * K + 16u * q;
+    const uint16_t* xrow = h + (size_t)t * stride + 8u * piece;
+    const uint16_t* erow = (eff ? eff : h) + 8u * piece;
+    h8 xv[CNT][2], ev[CNT][2];
+    u32x4 w[CNT];
+#pragma unroll
+    for (int c = 0; c < CNT; ++c) {
+        const uint32_t g = g0 + c < G ? g0 + c : G - 1;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            xv[c][u] = *reinterpret_cast<const h8*>(xrow + 64u * g + 32u * u);
+            ev[c][u] = *reinterpret_cast<const h8*>(erow + 64u * g + 32u * u);
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < CNT; ++c)
+        w[c] = *reinterpret_cast<const u32x4*>(wrow + 64u * (g0 + c < G ? g0 + c : G - 1));
+    copy_sb_to_lds<kQ8BlockThreads, 1>(m.s + (size_t)n0 * G, m.b + (size_t)n0 * G, sb, (E - n0 < 16u ? E - n0 : 16u) * G);
+    // x = h ⊙ eff, and the largest |x| of the slice (NaN aside) over the four lanes of the token
+    float x[CNT][2][8], top = 0.0f;
+#pragma unroll
+    for (int c = 0; c < CNT; ++c)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float v = (float)xv[c][u][i] * (eff ? (float)ev[c][u][i] : 1.0f);
+                x[c][u][i] = g0 + c < G ? v : 0.0f;
+                top = fmaxf(top, fabsf(x[c][u][i]));
+            }
+    top = rows_combine<true>(top);
+    // 2^k, k = 14 - exponent of the largest (a normal fp32 value: |x| is 0 or at least 2^-48)
+    const uint32_t ex = __builtin_bit_cast(uint32_t, top) >> 23;
+    const uint32_t kb = ex == 0 ? 127u : ex == 255u ? 127u - 17u : 127u + 14u + 127u - ex;
+    const float up = __builtin_bit_cast(float, kb << 23);
+    if (q == 0) inv[wave][r16] = __builtin_bit_cast(float, (254u - kb) << 23);
+    const uint32_t* sbt = sb + (row - n0) * G;
+    __syncthreads();
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    const h8 ones = {(_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f,
+                     (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f, (_Float16)1.0f};
+    // The codes are centred, q - 128 with bias b + 128·s: the same sum from
+    // terms that hardly cancel. INF: for tokens whose slice holds an infinity
+    // they stay 0..255, so that infinities and NaN arise where they do in the
+    // scalar form.
+    auto sum = [&](auto inf_c) {
+        constexpr bool INF = decltype(inf_c)::value;
+        f32x4 acc = zero;
+        const _Float16 base = (_Float16)(INF ? 1024.0f : 1152.0f);
+#pragma unroll
+        for (int c = 0; c < CNT; ++c) {
+            const auto p0 = __builtin_amdgcn_permlane32_swap(w[c].x, w[c].z, false, false);
+            const auto p1 = __builtin_amdgcn_permlane32_swap(w[c].y, w[c].w, false, false);
+            const h8 wv[2] = {q8_to_h8((uint32_t)p0[0], (uint32_t)p1[0], base),
+                              q8_to_h8((uint32_t)p0[1], (uint32_t)p1[1], base)};
+            f32x4 d = zero, sx = zero;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                h8 hi, lo;
+#pragma unroll
+                for (int i = 0; i < 8; i += 2) {
+                    // truncated to 11 bits each: the rest of a 22-bit value again has 11
+                    const float v0 = x[c][u][i] * up, v1 = x[c][u][i + 1] * up;
+                    const auto hp = __builtin_amdgcn_cvt_pkrtz(v0, v1);
+                    hi[i] = __builtin_bit_cast(h2, hp)[0];
+                    hi[i + 1] = __builtin_bit_cast(h2, hp)[1];
+                    float r0 = v0 - (float)hi[i], r1 = v1 - (float)hi[i + 1];
+                    if (INF) {
+                        r0 = __builtin_isfinite(v0) ? r0 : 0.0f;
+                        r1 = __builtin_isfinite(v1) ? r1 : 0.0f;
+                    }
+                    const auto lp = __builtin_amdgcn_cvt_pkrtz(r0, r1);
+                    lo[i] = __builtin_bit_cast(h2, lp)[0];
+                    lo[i + 1] = __builtin_bit_cast(h2, lp)[1];
+                }
+                d = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, wv[u], d, 0, 0, 0);
+                sx = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, ones, sx, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, wv[u], d, 0, 0, 0);
+                sx = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, ones, sx, 0, 0, 0);
+            }
+            const uint32_t tw = sbt[g0 + c < G ? g0 + c : G - 1];
+            const float sv = h2f((uint16_t)tw), bv = fmaf(INF ? 0.0f : 128.0f, sv, h2f((uint16_t)(tw >> 16)));
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[r] = fmaf(bv, sx[r], fmaf(sv, d[r], acc[r]));
+        }
+        return acc;
+    };
+    f32x4 acc = sum(std::false_type{});
+    if (__any(ex == 255u)) {
+        // opaque copies: nothing of the sum above is kept in registers for this rare one
+#pragma unroll
+        for (int c = 0; c < CNT; ++c) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(x[c][0][i]), "+v"(x[c][1][i]));
+            asm volatile("" : "+v"(w[c]));
+        }
+        const f32x4 a = sum(std::true_type{});
+        const uint64_t inf = __ballot(ex == 255u);        // bit t: token t (lanes 0..15)
+#pragma unroll
+        for (uint32_t r = 0; r < 4; ++r)
+            if ((inf >> (4u * q + r)) & 1u) acc[r] = a[r];
+    }
+    // back to the tokens' own scale, then the sum of the eight slices in wave order
+    acc *= *reinterpret_cast<const f32x4*>(&inv[wave][4u * q]);
+    red[wave][lane] = acc;
+    __syncthreads();
+    if (wave != 0) return;
+    f32x4 v = red[0][lane];
+#pragma unroll
+    for (uint32_t i = 1; i < kQ8BlockWaves; ++i) v += red[i][lane];
+#pragma unroll
+    for (uint32_t r = 0; r < 4; ++r)
+        if (n0 + r16 < E && t0 + 4u * q + r < T) logits[(size_t)(t0 + 4u * q + r) * E + n0 + r16] = v[r];
 }
 
 }  // namespace tfq

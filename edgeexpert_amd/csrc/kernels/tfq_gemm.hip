@@ -1,6 +1,6 @@
 // tfq_gemm.hip — the prefill dequant-fused GEMM: the 64-token MFMA projection tile
 // and the few-token weight stream, int4 and 3-bit, fp16 and bf16 activations; the
-// int8 rows over a block of tokens (shared expert).
+// int8 rows over a block of tokens (shared expert, router).
 #include "entry_points.hpp"
 #include "gemm_q8.hpp"
 
@@ -69,3 +69,13 @@ extern "C" __global__ __launch_bounds__(kQ8TileThreads, 2) void tfq_q8_tile_gate
                                                                                uint32_t ldx, uint32_t ldy) {
     gemm_q8_tile<true>(gate, up, X, Y, M, N, K, ldx, ldy);
 }
+
+// router logits of a block of tokens: C = ceil(d / 512) groups per wavefront
+#define TFQ_ROUTER_BLOCK(C)                                                                      \
+    extern "C" __global__ __launch_bounds__(kQ8BlockThreads, 2) void tfq_router_block_c##C(      \
+        Q8Mat m, const uint16_t* h, uint32_t stride, const uint16_t* eff, float* logits,         \
+        uint32_t T, uint32_t E, uint32_t K) {                                                    \
+        router_block<C>(m, h, stride, eff, logits, T, E, K);                                     \
+    }
+TFQ_ROUTER_BLOCK(1) TFQ_ROUTER_BLOCK(2) TFQ_ROUTER_BLOCK(3) TFQ_ROUTER_BLOCK(4)
+TFQ_ROUTER_BLOCK(5) TFQ_ROUTER_BLOCK(6) TFQ_ROUTER_BLOCK(7) TFQ_ROUTER_BLOCK(8)

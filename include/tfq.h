@@ -552,7 +552,9 @@ typedef struct {
 /* Router for a chunk of T tokens: hidden [T] rows of hidden_stride fp16
  * elements -> indices [T][top_k] and fp16 weights [T][top_k] (fp32 copy to
  * out_weights_f32 if non-NULL). logits_scratch: fp32 [T][num_experts].
- * Same arithmetic per token as tfq_router_topk. Replaces
+ * Per token the factored fp32 sums of tfq_router_topk; blocks of many tokens
+ * (16-byte aligned rows of hidden and effective_scale) form them on the matrix
+ * cores, every product exact, in another order of summation. Replaces
  * PrefillRouter.encodeGemma4Block (S/Kernels/Prefill/MoE/PrefillRouter.swift:37-89).
  * Contract: T >= 1, hidden_stride >= d, d % 64 == 0, d <= 4096,
  * 1 <= num_experts <= 256, 1 <= top_k <= min(64, num_experts). */

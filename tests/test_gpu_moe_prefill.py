@@ -56,6 +56,65 @@ def test_prefill_router_matches_per_token_reference(ctx, stream, T, E, D, k):
         assert oracle.rel_error(lg[t], ref_l) < 1e-5
 
 
+@pytest.mark.parametrize("T,E,D,with_eff,scale", [
+    (96, 128, 2816, True, 1.0), (97, 128, 64, False, 1.0), (130, 100, 704, True, 1e-4), (128, 256, 4096, True, 3e4),
+    (200, 65, 1088, False, 6e-6), (111, 112, 3648, True, 1.0)])
+def test_prefill_router_many_tokens(ctx, stream, T, E, D, with_eff, scale):
+    # many tokens take the matrix-core form: partial expert and token tiles,
+    # 1 .. 8 groups per wavefront (the last wavefronts with fewer or none),
+    # activations from fp16's subnormal range to its largest values. Logits
+    # against float64: the sums run over |s·q·x| + |b·x| terms whose fp32
+    # rounding (2^-24 each, ~sqrt(D) of them in any order) bounds the error.
+    W, S, B = synth.int8_matrix(3, f"prm/{E}x{D}", E, D)
+    H = synth.f16_bits(np.clip(synth.normal(synth.seed_key(3, f"prm/h{T}"), T * D) * np.float32(scale), -65504, 65504)
+                       ).reshape(T, D)
+    eff = synth.f16_bits(np.abs(synth.normal(synth.seed_key(3, "prm/eff"), D)) + 0.5) if with_eff else None
+    router = ops.Router(_dev(W), _dev(S), _dev(B), E, _dev(eff) if with_eff else None, None)
+    k = 8
+    idx, w16 = _dev(np.zeros(T * k, np.uint32)), _dev(np.zeros(T * k, np.uint16))
+    logits = _dev(np.zeros(T * E, np.float32))
+    ops.PrefillRouter(ctx).encode_gemma4_block(stream, router, _dev(H), D, T, D, k, idx, w16, logits)
+    stream.sync()
+    x = from_f16_bits(H).astype(np.float64) * (from_f16_bits(eff).astype(np.float64) if with_eff else 1.0)
+    s, b = from_f16_bits(S).astype(np.float64), from_f16_bits(B).astype(np.float64)
+    q = W.reshape(E, D // 64, 64).astype(np.float64)
+    ref = x @ (q * s[..., None] + b[..., None]).reshape(E, D).T
+    mass = np.abs(x) @ (q * np.abs(s)[..., None] + np.abs(b)[..., None]).reshape(E, D).T
+    got = logits.download(np.float32).reshape(T, E)
+    assert np.all(np.abs(got - ref) <= 2.0 ** -24 * 4 * mass)
+    # the selection is the per-token rule on these logits: value descending, index ascending
+    order = np.stack([np.lexsort((np.arange(E), -row)) for row in got])[:, :k]
+    assert np.array_equal(idx.download(np.uint32).reshape(T, k), order)
+
+
+def test_prefill_router_many_tokens_keeps_rows_apart(ctx, stream):
+    # rows with an infinity or NaN give the class of the per-token form (which
+    # a hidden that is only 2-byte aligned takes) and leave the other rows' bits
+    T, E, D, k = 96, 128, 512, 8
+    W, S, B = synth.int8_matrix(4, "prinf", E, D)
+    W[3] = 7                                          # no zero code and a positive bias: infinite, not NaN
+    B[3] = synth.f16_bits(np.full(D // 64, 0.5))
+    router = ops.Router(_dev(W), _dev(S), _dev(B), E, None, None)
+    H = synth.f16_vector(4, "prinf/h", T * D).reshape(T, D)
+    bad = H.copy()
+    bad[5, 100], bad[40, 3], bad[95, 511], bad[95, 0] = 0x7C00, 0x7E00, 0xFC00, 0x7BFF
+    out = []
+    for rows, off in ((H, 0), (bad, 0), (bad, 2)):
+        hb = DeviceBuffer(T * D * 2 + 16)
+        hb.upload(rows, offset=off)
+        idx, w16 = _dev(np.zeros(T * k, np.uint32)), _dev(np.zeros(T * k, np.uint16))
+        logits = _dev(np.zeros(T * E, np.float32))
+        ops.PrefillRouter(ctx).encode_gemma4_block(stream, router, hb.ptr(off), D, T, D, k, idx, w16, logits)
+        stream.sync()
+        out.append((logits.download(np.float32).reshape(T, E), idx.download(np.uint32).reshape(T, k)))
+    good = [t for t in range(T) if t not in (5, 40, 95)]
+    assert np.array_equal(out[0][0][good].view(np.uint32), out[1][0][good].view(np.uint32))
+    for t in (5, 40, 95):
+        a, b = out[1][0][t], out[2][0][t]
+        assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isposinf(a), np.isposinf(b))
+        assert np.array_equal(out[1][1][t], out[2][1][t])
+
+
 # ----------------------------------------------------------- grouping ----
 
 def _device_group(ctx, stream, idx, w16, T, k, E):
