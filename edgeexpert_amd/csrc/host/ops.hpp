@@ -1143,15 +1143,20 @@ public:
         e.log2_theta = epi.q_norm ? std::log2((double)epi.theta) : 0.0;
         char name[64];
         std::snprintf(name, sizeof(name), "tfq_attn_partial_h%u_g%u", hd, G);
-        void* a1[] = {&q, &k_cache, &v_cache, &nkv, &seq_len, &ks, &scale, &e, &part_o, &part_ml};
         hipFunction_t pf = m_.get(name);
         if (!pf) return fail(TFQ_E_NOT_LOADED, "kernel %s is not in the code object", name);
-        int rc = hip_check(hipModuleLaunchKernel(pf, nc, nkv, nsub, 256, 1, 1, 0, (hipStream_t)stream, a1, nullptr),
+        // one chunk per block while the GPU holds all blocks at once, else
+        // consecutive chunks per block so that it does
+        const uint64_t blocks = (uint64_t)nc * nkv * nsub, room = m_.resident_blocks(pf, 256, 0);
+        uint32_t cpb = (uint32_t)((blocks + room - 1) / room);
+        uint32_t nparts = (nc + cpb - 1) / cpb;
+        void* a1[] = {&q, &k_cache, &v_cache, &nkv, &seq_len, &ks, &scale, &e, &part_o, &part_ml, &nparts, &cpb};
+        int rc = hip_check(hipModuleLaunchKernel(pf, nparts * nkv * nsub, 1, 1, 256, 1, 1, 0, (hipStream_t)stream, a1,
+                                                 nullptr),
                            name);
         if (rc) return rc;
         std::snprintf(name, sizeof(name), "tfq_attn_combine_h%u", hd);
-        uint32_t ncu = nc;
-        void* a2[] = {&part_o, &part_ml, &out, &ncu};
+        void* a2[] = {&part_o, &part_ml, &out, &nparts};
         return launch2(m_, name, nq, hd / kAttnCombineDims, kAttnCombineThreads, 0, stream, a2);
     }
 

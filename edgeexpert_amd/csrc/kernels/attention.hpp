@@ -11,7 +11,13 @@
 // (m, l, O) in fp32. A second kernel merges the chunks of each query head:
 //     out[d] = fp16(Σ_c e^{m_c - M} O_c[d] / Σ_c e^{m_c - M} l_c),  M = max_c m_c,
 // which is the exact softmax of AttentionRef.apply
-// (V/Reference/Attention/Attention.swift:14-104) regrouped by chunk.
+// (V/Reference/Attention/Attention.swift:14-104) regrouped by chunk. When
+// there are more chunks than the GPU holds blocks, a block takes several
+// consecutive chunks as one part, rescaling its (l, O) to the new maximum
+// from chunk to chunk: one prologue and one partial row per part, and the
+// next chunk's K rows on their way during the current one's softmax and p·V.
+// 32768 keys per call, one chunk per block and here: 16 query / 2 kv heads of
+// 512 63.4 and 37.5 us, 16 / 8 heads of 256 69 and 52 us (floor 21 and 42).
 //
 // Mapping inside a block (256 threads): for q·k, 16 lanes own one key (each
 // lane HD/128 16-byte pieces of the row, so one load instruction covers
@@ -23,6 +29,8 @@
 // 16 q / 2 kv heads, two blocks of 4 heads each per (chunk, kv head), which
 // keeps the query registers to 64 per lane and gives 256 blocks at 4096 keys).
 #pragma once
+
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -84,23 +92,27 @@ struct AttnLds {
     uint16_t vp[HD];
     float rc[HD / 2];
     float rs[HD / 2];
-    float p[GB][kAttnChunk];
-    float ml[GB][2];
+    float p[2][GB][kAttnChunk];       // by chunk parity: the next scores are written while p·V still reads
+    float rescale[2][GB];
     float red[2048 / HD][GB][HD];
 };
 
-// One (chunk, kv head, query-head subset) block: blockIdx = (chunk, kv head h,
-// subset z), query heads h·G + z·GB + [0, GB). q: fp16 [num_q_heads][HD] (raw
-// projection when the epilogue is on); part_o: fp32
-// [num_q_heads][nchunks][HD]; part_ml: fp32 [num_q_heads][nchunks][2].
-// With GB < G every subset block of the new token's chunk runs the k/v
+// One (part, kv head, query-head subset) block: part blockIdx % nparts, the
+// chunks part·cpb .. of the keys, query heads h·G + z·GB + [0, GB). The
+// subset blocks of one (part, kv head) read the same K and V rows: blocks b
+// and b + 8 of the launch, which the dispatcher hands to the same XCD, so the
+// second finds them in its L2. q: fp16 [num_q_heads][HD] (raw projection when
+// the epilogue is on); part_o: fp32 [num_q_heads][nparts][HD]; part_ml: fp32
+// [num_q_heads][nparts][2].
+// With GB < G every subset block of the new token's part runs the k/v
 // epilogue on the staged raw rows (epi.k_raw / v_raw) and writes the same
 // words into the cache slot; nothing reads that slot from the caches.
 template <int HD, int G, int GB = G>
 __device__ __forceinline__ void attn_partial(const uint16_t* __restrict__ q, uint16_t* __restrict__ kc,
                                              uint16_t* __restrict__ vc, uint32_t nkv, uint32_t seq_len,
                                              uint32_t kv_start, float scale, const AttnEpilogue& epi,
-                                             float* __restrict__ part_o, float* __restrict__ part_ml) {
+                                             float* __restrict__ part_o, float* __restrict__ part_ml,
+                                             uint32_t nparts, uint32_t cpb) {
     static_assert(HD == 128 || HD == 256 || HD == 512, "head_dim 128, 256 or 512");
     static_assert(GB >= 1 && G % GB == 0, "query heads split evenly over blocks");
     constexpr uint32_t CPL = HD / 128;                 // 16-byte pieces per lane per key (q·k)
@@ -111,16 +123,30 @@ __device__ __forceinline__ void attn_partial(const uint16_t* __restrict__ q, uin
     __shared__ __attribute__((aligned(16))) AttnLds<HD, GB> L;
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t chunk = blockIdx.x, h = blockIdx.y, nchunks = gridDim.x;
-    const uint32_t qh0 = h * G + (GB < G ? blockIdx.z * GB : 0u);       // first query head of the block
-    const uint32_t c0 = kv_start + chunk * kAttnChunk;
-    const uint32_t n = seq_len - c0 < kAttnChunk ? seq_len - c0 : kAttnChunk;
+    constexpr uint32_t NSUB = G / GB;
+    // (part, kv head) unit and subset of this block
+    uint32_t unit = blockIdx.x, sub = 0;
+    if constexpr (NSUB > 1) {
+        const uint32_t whole = nparts * nkv & ~7u;        // units in full groups of 8 XCDs
+        if (unit < NSUB * whole) {
+            sub = (unit >> 3) % NSUB;
+            unit = (unit >> 3) / NSUB * 8u + (unit & 7u);
+        } else {
+            sub = (unit - NSUB * whole) % NSUB;
+            unit = whole + (unit - NSUB * whole) / NSUB;
+        }
+    }
+    const uint32_t part = unit % nparts, h = unit / nparts;
+    const uint32_t qh0 = h * G + sub * GB;                               // first query head of the block
+    const uint32_t nchunks = (seq_len - kv_start + kAttnChunk - 1) / kAttnChunk;
+    const uint32_t ch0 = part * cpb, ch1 = ch0 + cpb < nchunks ? ch0 + cpb : nchunks;   // this part's chunks
     const size_t row = (size_t)nkv * HD;               // halves between consecutive positions
-    const uint16_t* kbase = kc + (size_t)c0 * row + (size_t)h * HD;
-    const uint16_t* vbase = vc + (size_t)c0 * row + (size_t)h * HD;
+    const uint16_t* kbase = kc + (size_t)kv_start * row + (size_t)h * HD;
+    const uint16_t* vbase = vc + (size_t)kv_start * row + (size_t)h * HD;
     const bool epi_on = epi.q_norm != nullptr;
     const uint32_t pos = seq_len - 1;                  // the new token
-    const bool own_pos = epi_on && pos >= c0 && pos < c0 + n;
+    const bool own_pos = epi_on && ch1 == nchunks;     // the last part holds it
+    const uint32_t span = seq_len - kv_start;          // visible keys
 
     // 1. loads, in the order they are waited for: the queries (16-byte
     // chunks; G*HD/8 <= 256 of them), the norm weights and, in the block that
@@ -143,15 +169,16 @@ __device__ __forceinline__ void attn_partial(const uint16_t* __restrict__ q, uin
     const uint4 wraw = reinterpret_cast<const uint4*>(wsrc)[kvi % (HD / 8)];
 
     const uint32_t sl = lane & (kAttnKeyLanes - 1);
-    uint4 kr[KSTEPS][CPL];
-#pragma unroll
-    for (uint32_t st = 0; st < KSTEPS; ++st) {
-        const uint32_t j = st * (kAttnThreads / kAttnKeyLanes) + (tid >> 4);
-        const uint32_t jr = j < n ? j : n - 1;
+    u32x4 kr[KSTEPS][CPL];
+    auto load_k = [&](uint32_t ch, uint32_t st) {
+        const uint32_t j = ch * kAttnChunk + st * (kAttnThreads / kAttnKeyLanes) + (tid >> 4);
+        const uint32_t jr = j < span ? j : span - 1;
 #pragma unroll
         for (uint32_t cc = 0; cc < CPL; ++cc)
-            kr[st][cc] = *reinterpret_cast<const uint4*>(kbase + jr * row + 8u * (sl + 16u * cc));
-    }
+            kr[st][cc] = *reinterpret_cast<const u32x4*>(kbase + jr * row + 8u * (sl + 16u * cc));
+    };
+#pragma unroll
+    for (uint32_t st = 0; st < KSTEPS; ++st) load_k(ch0, st);
     // 2. queries (and the new token's k/v) through the epilogue
     if (tid < QCH) reinterpret_cast<uint4*>(&L.q[0][0])[tid] = qraw;
     if (epi_on) {
@@ -186,87 +213,116 @@ __device__ __forceinline__ void attn_partial(const uint16_t* __restrict__ q, uin
         __syncthreads();
     }
 
-    // the chunk's V rows, issued after the epilogue: a wave stalls while the
-    // memory pipeline backs up under its loads, so the epilogue runs under
-    // the K stream (which alone keeps HBM busy) instead of after both
     const uint32_t vg = tid / TPR, vl = tid % TPR;
-    uint4 vr[KPG];
-#pragma unroll
-    for (uint32_t i = 0; i < KPG; ++i) {
-        const uint32_t j = vg * KPG + i;
-        vr[i] = *reinterpret_cast<const uint4*>(vbase + (j < n ? j : n - 1) * row + 8u * vl);
-    }
-
-    // 3. scores
-    h2 qv[GB][CPL][4];
-#pragma unroll
-    for (int g = 0; g < GB; ++g)
-#pragma unroll
-        for (uint32_t cc = 0; cc < CPL; ++cc) {
-            const uint4 raw = *reinterpret_cast<const uint4*>(&L.q[g][8u * (sl + 16u * cc)]);
-            qv[g][cc][0] = __builtin_bit_cast(h2, raw.x);
-            qv[g][cc][1] = __builtin_bit_cast(h2, raw.y);
-            qv[g][cc][2] = __builtin_bit_cast(h2, raw.z);
-            qv[g][cc][3] = __builtin_bit_cast(h2, raw.w);
-        }
-#pragma unroll
-    for (uint32_t st = 0; st < KSTEPS; ++st) {
-        const uint32_t j = st * (kAttnThreads / kAttnKeyLanes) + (tid >> 4);
-        float acc[GB];
-#pragma unroll
-        for (int g = 0; g < GB; ++g) acc[g] = 0.0f;
-#pragma unroll
-        for (uint32_t cc = 0; cc < CPL; ++cc) {
-            uint4 kk = kr[st][cc];
-            if (own_pos && c0 + j == pos) kk = *reinterpret_cast<const uint4*>(&L.kp[8u * (sl + 16u * cc)]);
-            const h2 k4[4] = {__builtin_bit_cast(h2, kk.x), __builtin_bit_cast(h2, kk.y),
-                              __builtin_bit_cast(h2, kk.z), __builtin_bit_cast(h2, kk.w)};
-#pragma unroll
-            for (int g = 0; g < GB; ++g)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[g] = __builtin_amdgcn_fdot2(k4[e], qv[g][cc][e], acc[g], false);
-        }
-#pragma unroll
-        for (int g = 0; g < GB; ++g) {
-            const float sdot = row16_sum(acc[g]);
-            if (sl == 0) L.p[g][j] = j < n ? sdot * scale : -__builtin_inff();
-        }
-    }
-    __syncthreads();
-
-    // 4. chunk softmax statistics, one wavefront per query head
-    for (uint32_t g = wave; g < (uint32_t)GB; g += kAttnThreads / 64) {
-        const float sv = lane < kAttnChunk ? L.p[g][lane] : -__builtin_inff();
-        const float m = wave_max(sv);
-        const float e = lane < n ? expf(sv - m) : 0.0f;
-        const float l = wave_sum(e);
-        if (lane < kAttnChunk) L.p[g][lane] = e;
-        if (lane == 0) {
-            L.ml[g][0] = m;
-            L.ml[g][1] = l;
-        }
-    }
-    __syncthreads();
-
-    // 5. p·V
     float o[GB][8];
 #pragma unroll
     for (int g = 0; g < GB; ++g)
 #pragma unroll
         for (int e = 0; e < 8; ++e) o[g][e] = 0.0f;
+    // from head_dim 256 on the next chunk's K rows are requested as p·V frees
+    // the registers of the V rows: both sets at once spill at head_dim 512 (93
+    // us for 32768 keys), and cost 256 about 2%
+    constexpr bool LATE_K = HD >= 256;
+    float m_run = -__builtin_inff(), l_run = 0.0f;       // of query head `wave` (waves below GB)
+    static_assert(GB <= kAttnThreads / 64, "one wavefront per query head");
+
+    // 3.-5. of one chunk: scores, softmax statistics, p·V
+    auto chunk = [&](uint32_t ch, auto more_c) {
+        constexpr bool MORE = decltype(more_c)::value;    // another chunk follows
+        const uint32_t k0 = ch * kAttnChunk, par = ch & 1u;
+        const uint32_t n = span - k0 < kAttnChunk ? span - k0 : kAttnChunk;
+        // the chunk's V rows, issued after the epilogue: a wave stalls while the
+        // memory pipeline backs up under its loads, so the epilogue runs under
+        // the K stream (which alone keeps HBM busy) instead of after both
+        u32x4 vr[KPG];
 #pragma unroll
-    for (uint32_t i = 0; i < KPG; ++i) {
-        const uint32_t j = vg * KPG + i;
-        uint4 vv = vr[i];
-        if (own_pos && c0 + j == pos) vv = *reinterpret_cast<const uint4*>(&L.vp[8u * vl]);
-        const h8 v8 = __builtin_bit_cast(h8, vv);
-#pragma unroll
-        for (int g = 0; g < GB; ++g) {
-            const float pj = L.p[g][j];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) o[g][e] = fmaf(pj, (float)v8[e], o[g][e]);
+        for (uint32_t i = 0; i < KPG; ++i) {
+            const uint32_t j = k0 + vg * KPG + i;
+            vr[i] = *reinterpret_cast<const u32x4*>(vbase + (j < span ? j : span - 1) * row + 8u * vl);
         }
-    }
+        // the queries of one 128-dim piece at a time (from LDS: kept in
+        // registers over the chunks they would take GB·HD/32 of them)
+        float acc[KSTEPS][GB];
+#pragma unroll
+        for (uint32_t st = 0; st < KSTEPS; ++st)
+#pragma unroll
+            for (int g = 0; g < GB; ++g) acc[st][g] = 0.0f;
+#pragma unroll
+        for (uint32_t cc = 0; cc < CPL; ++cc) {
+            u32x4 qv[GB];
+#pragma unroll
+            for (int g = 0; g < GB; ++g) qv[g] = *reinterpret_cast<const u32x4*>(&L.q[g][8u * (sl + 16u * cc)]);
+#pragma unroll
+            for (uint32_t st = 0; st < KSTEPS; ++st) {
+                const uint32_t j = st * (kAttnThreads / kAttnKeyLanes) + (tid >> 4);
+                u32x4 kk = kr[st][cc];
+                if (own_pos && kv_start + k0 + j == pos) kk = *reinterpret_cast<const u32x4*>(&L.kp[8u * (sl + 16u * cc)]);
+#pragma unroll
+                for (int g = 0; g < GB; ++g)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        acc[st][g] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, (uint32_t)kk[e]),
+                                                            __builtin_bit_cast(h2, (uint32_t)qv[g][e]), acc[st][g], false);
+            }
+        }
+#pragma unroll
+        for (uint32_t st = 0; st < KSTEPS; ++st) {
+            const uint32_t j = st * (kAttnThreads / kAttnKeyLanes) + (tid >> 4);
+#pragma unroll
+            for (int g = 0; g < GB; ++g) {
+                const float sdot = row16_sum(acc[st][g]);
+                if (sl == 0) L.p[par][g][j] = j < n ? sdot * scale : -__builtin_inff();
+            }
+        }
+        if (MORE && !LATE_K)
+#pragma unroll
+            for (uint32_t st = 0; st < KSTEPS; ++st) load_k(ch + 1, st);
+        __syncthreads();
+
+        // one wavefront per query head
+        if (wave < (uint32_t)GB) {
+            const uint32_t g = wave;
+            const float sv = L.p[par][g][lane];
+            const float m = fmaxf(m_run, wave_max(sv));
+            const float e = lane < n ? expf(sv - m) : 0.0f;
+            const float r = ch == ch0 ? 0.0f : expf(m_run - m);
+            l_run = ch == ch0 ? wave_sum(e) : fmaf(l_run, r, wave_sum(e));
+            m_run = m;
+            L.p[par][g][lane] = e;
+            if (lane == 0) L.rescale[par][g] = r;
+        }
+        __syncthreads();
+
+        if (ch != ch0) {
+#pragma unroll
+            for (int g = 0; g < GB; ++g) {
+                const float r = L.rescale[par][g];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[g][e] *= r;
+            }
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < KPG; ++i) {
+            const uint32_t j = vg * KPG + i;
+            u32x4 vv = vr[i];
+            if (own_pos && kv_start + k0 + j == pos) vv = *reinterpret_cast<const u32x4*>(&L.vp[8u * vl]);
+            const h8 v8 = __builtin_bit_cast(h8, vv);
+#pragma unroll
+            for (int g = 0; g < GB; ++g) {
+                const float pj = L.p[par][g][j];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[g][e] = fmaf(pj, (float)v8[e], o[g][e]);
+            }
+            if (LATE_K && i % (KPG / KSTEPS) == KPG / KSTEPS - 1) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (MORE) load_k(ch + 1, i / (KPG / KSTEPS));
+            }
+        }
+    };
+    uint32_t ch = ch0;
+    for (; ch + 1 < ch1; ++ch) chunk(ch, std::true_type{});
+    chunk(ch, std::false_type{});
+
 #pragma unroll
     for (int g = 0; g < GB; ++g)
 #pragma unroll
@@ -278,12 +334,12 @@ __device__ __forceinline__ void attn_partial(const uint16_t* __restrict__ q, uin
 #pragma unroll
         for (uint32_t r = 0; r < VGROUPS; ++r) s += L.red[r][g][d];
         const size_t qh = (size_t)qh0 + g;
-        part_o[(qh * nchunks + chunk) * HD + d] = s;
+        part_o[(qh * nparts + part) * HD + d] = s;
     }
-    if (tid < (uint32_t)GB) {
-        const size_t qh = (size_t)qh0 + tid;
-        part_ml[(qh * nchunks + chunk) * 2 + 0] = L.ml[tid][0];
-        part_ml[(qh * nchunks + chunk) * 2 + 1] = L.ml[tid][1];
+    if (wave < (uint32_t)GB && lane == 0) {
+        const size_t qh = (size_t)qh0 + wave;
+        part_ml[(qh * nparts + part) * 2 + 0] = m_run;
+        part_ml[(qh * nparts + part) * 2 + 1] = l_run;
     }
 }
 

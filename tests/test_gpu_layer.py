@@ -71,6 +71,36 @@ def test_attention_matches_reference(ctx, stream, hd, nq, nkv, seq, window, scal
     assert rel < TOL, f"{tag}: rel={rel}"
 
 
+@pytest.mark.parametrize("hd,nq,nkv,seq,window", [
+    (512, 16, 2, 8257, 0),       # two chunks per block, the last block with one of one key
+    (512, 16, 2, 24700, 0),      # four chunks, the last block with two, ragged
+    (256, 32, 8, 5000, 0),       # group 4
+    (256, 16, 8, 12400, 0),      # group 2
+    (256, 16, 8, 30000, 6500),   # a window of more chunks than the GPU holds blocks
+    (128, 16, 8, 13000, 0),
+    (512, 8, 8, 4200, 0),        # group 1
+])
+@pytest.mark.parametrize("spike", [False, True])
+def test_attention_several_chunks_per_block(ctx, stream, hd, nq, nkv, seq, window, spike):
+    # more 64-key chunks than resident blocks: a block runs consecutive chunks
+    # and rescales its partial sums to each new maximum. spike: keys that
+    # dominate at the start, in the middle and at the end of the sequence, so
+    # that maxima both rise and stay between a block's chunks
+    tag = f"attnm-h{hd}-q{nq}-kv{nkv}-T{seq}-w{window}"
+    q16 = synth.f16_vector(0, tag + "/q", nq * hd)
+    k16 = synth.f16_vector(0, tag + "/k", seq * nkv * hd).reshape(seq, nkv, hd)
+    v16 = synth.f16_vector(0, tag + "/v", seq * nkv * hd)
+    if spike:
+        qf = from_f16_bits(q16).reshape(nkv, nq // nkv, hd)
+        for j, s in ((seq - 1, 0.02), (seq // 2, 0.05), (seq - (window or seq) + 3, 0.03)):
+            k16[j] = synth.f16_bits(qf[:, 0] * s * np.sqrt(hd) / 2)
+    got = _run_attention(ctx, stream, q16, k16, v16, hd, nq, nkv, seq, window, None)
+    ref = oracle.attention(from_f16_bits(q16), from_f16_bits(k16.reshape(-1)), from_f16_bits(v16), hd, nq, nkv, seq,
+                           window, None)
+    rel = oracle.rel_error(got, ref)
+    assert rel < TOL, f"{tag}: rel={rel}"
+
+
 def test_attention_is_deterministic(ctx, stream):
     hd, nq, nkv, seq = 256, 16, 8, 2048
     q16 = synth.f16_vector(1, "det/q", nq * hd)
@@ -288,6 +318,16 @@ CONFIG4_FULL = dict(CONFIG4, nkv=2, hd=512, rotated_pairs=64, theta=1e6, full=Tr
 def test_layer_small_full_attention(ctx, stream, pos):
     got, ref, w, hid = _layer_case(ctx, stream, SMALL_FULL, 8, pos, 160, 10, f"small-full-{pos}")
     _check_layer(got, ref, w, SMALL_FULL, hid, f"small full pos={pos}")
+
+
+@pytest.mark.parametrize("full", [True, False])
+def test_layer_small_several_chunks_per_block(ctx, stream, full):
+    # the new token in the last of a block's several chunks: the staged k/v of
+    # the full form (both query subsets), the cache slot of the sliding form
+    shape = SMALL_FULL if full else dict(SMALL, nq=16, nkv=8, hd=256, rotated_pairs=128)
+    pos = 16450 if full else 6210
+    got, ref, w, hid = _layer_case(ctx, stream, shape, 8, pos, pos + 1, 12, f"small-long-{full}")
+    _check_layer(got, ref, w, shape, hid, f"small long full={full}")
 
 
 def test_layer_config4_full_attention(ctx, stream):
