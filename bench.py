@@ -597,7 +597,7 @@ def layer_summary(trace_csv, out=sys.stdout):
 def bench_gemm_policy(ctx, stream, batch_avg_us):
     """The prefill GEMM's kernel choice by token count (config 2's weights,
     N 8192 x K 2816, bf16): the library's choice at token counts on both
-    sides of its crossover (80 tokens at this N), and both kernels forced at
+    sides of its crossover (112 tokens at this N), and both kernels forced at
     the two counts next to it."""
     from edgeexpert_amd import ops, synth
     from edgeexpert_amd._lib import DTYPE_BF16, GEMM_PATH_SKINNY32, GEMM_PATH_TILE
@@ -610,7 +610,7 @@ def bench_gemm_policy(ctx, stream, batch_avg_us):
     Y = DeviceBuffer(512 * N * 2)
     q = ops.PrefillInt4QMM(ctx)
     wbytes = N * Kd // 2 + 2 * N * (Kd // 64) * 2
-    out = {"shape": [None, N, Kd], "crossover_tokens": 80, "auto": {}, "forced": {}}
+    out = {"shape": [None, N, Kd], "crossover_tokens": 112, "auto": {}, "forced": {}}
 
     def run(m, path):
         return batch_avg_us(lambda i: q.encode(stream, *bufs[i % copies], X, Y, m, N, Kd, DTYPE_BF16, path=path),
@@ -619,7 +619,7 @@ def bench_gemm_policy(ctx, stream, batch_avg_us):
         us = run(m, None)
         out["auto"][str(m)] = {"us": round(us, 2), "tflops": round(2.0 * m * N * Kd / (us * 1e-6) / 1e12, 1),
                                "weight_gbs": round(wbytes / (us * 1e-6) / 1e9, 1),
-                               "kernel": "gemv" if m == 1 else "skinny" if m <= 80 else "tile"}
+                               "kernel": "gemv" if m == 1 else "skinny" if m <= 112 else "tile"}
     for m in (64, 96):
         out["forced"][str(m)] = {"skinny32_us": round(run(m, GEMM_PATH_SKINNY32), 2),
                                  "tile_us": round(run(m, GEMM_PATH_TILE), 2)}

@@ -756,37 +756,37 @@ constexpr uint32_t kSkinnyThreads = 512;    // (gemm_skinny.hpp kSkinnyThreads)
 // token tile). Both multiply the same fp16 weights, so the choice changes
 // time, not results beyond fp32 summation order. The skinny form is used up
 // to the largest token count at which it measured faster on MI355X for that
-// output count (K = 2816; see skinny_max_tokens).
+// output count (see skinny_max_tokens).
 struct GemmPlan {
     int path;        // TFQ_GEMM_PATH_TILE, _SKINNY (16 rows per wave) or _SKINNY32 (32)
 };
 
 // Largest token count at which the weight stream beat the tile on MI355X
-// (bf16 activations, K = 2816, back-to-back launches; the tile takes ~28 us
-// at any token count up to 448 at these shapes, the stream grows by one
-// weight pass per 16 tokens): N = 2048: 320, 2816: 192, 4096: 160, 8192: 80.
-// Other N follow the measured ~1/N trend. The crossover is taken to be
-// independent of K: both kernels' times scale with K.
+// (back-to-back launches, cold weights). The stream takes ~4 us and 7.7e-9 us
+// per token, output and input (8192 x 2816 at 64 / 128 / 256 tokens: 15.4,
+// 26.8, 49.6 us; 2816 x 4096: 12.4, 17.5, 29.2; 2048 x 2816: 6.1, 8.6, 14.3);
+// the tile takes ~0.0085 us per input while its blocks fit the GPU at once
+// (24 us at 2816 inputs, 42 at 4096, 9 at 704), whatever the tokens. Both
+// scale with the inputs, so the crossover is one over the outputs: measured
+// 112 tokens at 8192 outputs, ~450 at 2048, ~300 at 2816 x 704, ~400 at 2816 x 4096.
 inline uint32_t skinny_max_tokens(uint32_t n, uint32_t k) {
     (void)k;
-    if (n <= 2048) return 320;
-    if (n <= 2816) return 192;
-    if (n <= 4096) return 160;
-    if (n <= 8192) return 80;
-    const uint32_t t = 655360u / n / 16u * 16u;
+    const uint32_t t = 917504u / n / 16u * 16u;
     return t < 16 ? 16 : t;
 }
 
 inline GemmPlan plan_gemm(uint32_t t, uint32_t n, uint32_t k) {
-    // one token: the decode GEMV (N 2048: 3.9 against 4.4 us for the weight
-    // stream, N 8192: 5.8 against 6.4 us, cold weights); from two tokens on
+    // one token: the decode GEMV (N 2048: 3.9 against 4.2 us for the weight
+    // stream, N 8192: 5.8 against 6.3 us, cold weights); from two tokens on
     // the stream reads the weights once for up to 16 tokens and wins (N 8192,
-    // two tokens: 6.5 against 11.2 us for two GEMVs)
+    // two tokens: 6.3 against 11.2 us for two GEMVs)
     if (t == 1) return {TFQ_GEMM_PATH_GEMV};
     if (t > skinny_max_tokens(n, k)) return {TFQ_GEMM_PATH_TILE};
-    // 16 rows per wave keeps more blocks for narrow matrices and few tokens;
-    // 32 rows per wave halves the activation reads and wins elsewhere
-    const bool rows16 = (t <= 16 && n < 8192) || (t <= 32 && n <= 2048);
+    // 16 rows per wave while that gives at most one block per CU (2816 x 4096,
+    // 16 tokens: 5.8 against 8.9 us for 32 rows), else 32 rows, which read the
+    // activations half as often (8192 x 2816, 64 tokens: 15.4 against 17.8 us;
+    // between one and three blocks per CU the two are within 5%)
+    const bool rows16 = (uint64_t)((n + 15) / 16) * ((t + 15) / 16) <= 256;
     return {rows16 ? TFQ_GEMM_PATH_SKINNY : TFQ_GEMM_PATH_SKINNY32};
 }
 

@@ -171,8 +171,9 @@ __device__ __forceinline__ DequantConsts<BITS> dequant_consts() {
     return dc;
 }
 
-// Word j of a chunk (codes 8j..8j+7) dequantised as fp16(q·s + b) with one
-// rounding, s and b from one table word (scale | bias << 16). 4 bits: each
+// A block word (block_word: 8 codes) dequantised as fp16(q·s + b) with one
+// rounding, s and b from one word (scale | bias << 16); dequant_word_sb: word
+// j of a chunk (codes 8j..8j+7). 4 bits: each
 // code lands in the low nibble of a byte (word & 0x0F0F0F0F and its shift by
 // 4), which read as an FP8 E4M3 number is q·2^-9 exactly (q < 8: subnormal
 // q·2^-9; q >= 8: exponent field 1, (8 + (q-8))·2^-9); the gfx950
@@ -181,10 +182,9 @@ __device__ __forceinline__ DequantConsts<BITS> dequant_consts() {
 // (unit_b_order). 2 and 3 bits: the fields of DqField, in the order
 // (0,4,1,5,2,6,3,7).
 template <int BITS>
-__device__ __forceinline__ h8 dequant_word_sb(const QChunk<BITS>& w, int j, uint32_t sb, const DequantConsts<BITS>& dc) {
+__device__ __forceinline__ h8 dequant_block_sb(uint32_t t, uint32_t sb, const DequantConsts<BITS>& dc) {
     const h2 s2 = __builtin_bit_cast(h2, __builtin_amdgcn_perm(sb, sb, 0x01000100u));
     const h2 b2 = __builtin_bit_cast(h2, __builtin_amdgcn_perm(sb, sb, 0x03020302u));
-    uint32_t t = block_word<BITS>(w, j);
     h8 run;
     if constexpr (BITS == 4) {
         const uint32_t lo = t & 0x0F0F0F0Fu, hi = (t >> 4) & 0x0F0F0F0Fu;
@@ -213,6 +213,10 @@ __device__ __forceinline__ h8 dequant_word_sb(const QChunk<BITS>& w, int j, uint
         }
     }
     return run;
+}
+template <int BITS>
+__device__ __forceinline__ h8 dequant_word_sb(const QChunk<BITS>& w, int j, uint32_t sb, const DequantConsts<BITS>& dc) {
+    return dequant_block_sb<BITS>(block_word<BITS>(w, j), sb, dc);
 }
 
 // The activation order that matches dequant_word_sb's code order.
