@@ -1012,30 +1012,28 @@ public:
                         kGroupMaxTiles);
         ExpertPool kp = kernel_pool(pool);
         // one launch per projection over the work list of the tiles: tiles of
-        // at most 32 pairs as stream units (RT 4: 128 features / 256 outputs
-        // per unit, NTT 1 or 2 pair sub-tiles), larger ones as 64-pair halves
-        // on wide units (RT 2: 64 features / 128 outputs, NTT 2 or 4); the
+        // at most 32 pairs as stream units, larger ones as 64-pair halves on
+        // wide units (64 features / 128 outputs per unit either way); the
         // grid is the blocks the GPU holds resident, at most the units the
         // tile bound allows
         const uint32_t bits = pool_bits(pool);
         // the _t launches stage each unit's scale/bias table through
         // registers: 16-byte aligned scale/bias arrays (base and stride are)
-        // whose unit tables fit (d <= 3072 for gate/up, f <= 1024 for down)
+        // whose unit tables fit (d <= 4096 for gate/up, f <= 1024 for down)
         const tfq_expert_offsets& po = pool.offsets;
         bool sb16 = true;
         for (uint64_t v : {po.gate_s, po.gate_b, po.up_s, po.up_b, po.down_s, po.down_b}) sb16 = sb16 && v % 16 == 0;
         // (moe_prefill.hpp TableRegs: rows·K/64 words in U 16-byte pieces per thread)
         auto fits = [](uint32_t rows, uint32_t K, uint32_t U) { return rows * (K / 64u) <= 8u * U * kUnitThreads; };
-        const bool tab_gu = sb16 && fits(128, d, 3), tab_dn = sb16 && fits(256, f, 2);
+        const bool tab_gu = sb16 && fits(64, d, 2), tab_dn = sb16 && fits(128, f, 1);
         char gu[48], dn[48];
         const char* bsuf = bits == 2 ? "_b2" : bits == 3 ? "_b3" : "";
         std::snprintf(gu, sizeof(gu), "tfq_moe_grouped_gate_up%s%s", bsuf, tab_gu ? "_t" : "");
         std::snprintf(dn, sizeof(dn), "tfq_moe_grouped_down%s%s", bsuf, tab_dn ? "_t" : "");
-        // dynamic LDS: the largest unit (two activation buffers of 16·NTT
-        // rows, then the table of 64·RT rows of K/64 words)
+        // dynamic LDS: the largest unit (two activation buffers of 64 pairs,
+        // then the table of 128 rows of K/64 words)
         auto lds_for = [](uint32_t K) {
-            auto unit = [K](uint32_t rt, uint32_t ntt) { return 2u * 16u * ntt * kUnitStride * 2u + 4u * 64u * rt * (K / 64u); };
-            return std::max(unit(2, 4), unit(4, 2));
+            return 2u * 64u * kUnitStride * 2u + 4u * 128u * (K / 64u);
         };
         auto grid_for = [&](const char* name, const GroupedLaunch& g, uint32_t lds, uint32_t& grid) {
             hipFunction_t fn = m_.get(name);
@@ -1045,14 +1043,14 @@ public:
             grid = std::min(p, units);
             return TFQ_OK;
         };
-        GroupedLaunch g1{max_tiles, (f + 63) / 64, (f + 127) / 128};
+        GroupedLaunch g1{max_tiles, (f + 63) / 64, (f + 63) / 64};
         uint32_t grid1 = 0, grid2 = 0;
         rc = grid_for(gu, g1, lds_for(d), grid1);
         if (rc) return rc;
         void* a1[] = {&kp, &sorted, &tiles, &n_tiles, &hidden, &stride, &act, &d, &f, &g1};
         rc = launch2(m_, gu, grid1, 1, kUnitThreads, lds_for(d), stream, a1);
         if (rc) return rc;
-        GroupedLaunch g2{max_tiles, (d + 127) / 128, (d + 255) / 256};
+        GroupedLaunch g2{max_tiles, (d + 127) / 128, (d + 127) / 128};
         rc = grid_for(dn, g2, lds_for(f), grid2);
         if (rc) return rc;
         void* a2[] = {&kp, &sorted, &tiles, &n_tiles, &act, &partials, &d, &f, &k, &g2};

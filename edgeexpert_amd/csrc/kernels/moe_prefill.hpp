@@ -251,15 +251,15 @@ __device__ __forceinline__ void sfor_while(Fn&& f) {
 // 64-pair half of a tile of more than kGroupStreamMax pairs, or a whole
 // smaller tile) times a block of weight rows. Each of the four wavefronts owns
 // RT 16-row A operands of v_mfma_f32_16x16x32_f16 and the whole K loop; the
-// pairs are NTT 16-pair B operands. Two shapes:
-//   wide   (tiles of more than 32 pairs): RT 2, NTT 2 or 4, 128 rows per unit
-//          (gate/up: 64 features, gate and up rows; down: 128 outputs);
-//   stream (tiles of at most 32 pairs):   RT 4, NTT 1 or 2, 256 rows per unit
-//          (gate/up: 128 features; down: 256 outputs).
-// Under a skewed popularity most experts see a handful of tokens (config 3:
-// 101 of 128 experts take at most 32 of the 4096 pairs, yet hold 80% of the
-// active weights), so the stream shape spreads each activation k-tile over
-// twice the rows. Lane l holds row l%16 of each A operand and the quarter
+// pairs are NTT 16-pair B operands: RT 2, 128 rows per unit (gate/up: 64
+// features, gate and up rows; down: 128 outputs) for wide units (tiles of more
+// than 32 pairs, NTT 2 or 4) and stream units (the others, NTT 1 or 2) alike.
+// Stream units of 256 rows (RT 4) spread an activation k-tile over twice the
+// rows but are too few to share out evenly over the blocks: 33 tokens of a
+// 128-expert block are ~530 gate/up units of them on 512 blocks, two rounds
+// with the second nearly empty, and 704 features leave the last one half
+// empty. With 128 rows: 512 tokens at 4 bits 203.3 -> 195.5 us per call, 33
+// tokens at 3 bits 107.2 -> 101.9. Lane l holds row l%16 of each A operand and the quarter
 // q = l/16 of every 128-code k-tile (chunk 4m + q: one 16-byte load at 4 bits;
 // word u feeds k-step u), dequantised from a DEPTH-deep register ring with the
 // scale and bias of an LDS table (one word per row and group). The unit's
@@ -437,9 +437,7 @@ __device__ __forceinline__ void unit_rows_loop(const uint8_t* const (&wbase)[RT]
     });
 }
 
-// ring depth of a shape: the 64-row waves hold four k-tiles of weights
-template <int RT>
-constexpr int unit_depth() { return RT == 2 ? 3 : 4; }
+constexpr int kUnitDepth = 3;                // k-tiles of weights in the ring
 
 // Gate/up + GeGLU of one unit over 32·RT features (row block bx): wave w
 // takes features f_blk + 16·(RT/2)·w + (0..16·RT/2-1), its gate rows as row
@@ -480,8 +478,8 @@ __device__ __forceinline__ void unit_gate_up(const ExpertPool& pool, const Pair*
     const uint16_t* gb = reinterpret_cast<const uint16_t*>(blob + o.gate_b) + (size_t)f_blk * G;
     const uint16_t* us = reinterpret_cast<const uint16_t*>(blob + o.up_s) + (size_t)f_blk * G;
     const uint16_t* ub = reinterpret_cast<const uint16_t*>(blob + o.up_b) + (size_t)f_blk * G;
-    TableRegs<TAB ? (RT == 4 ? 3u : 2u) : 1u> tg, tu;
-    unit_rows_loop<BITS, RT, NTT, unit_depth<RT>()>(
+    TableRegs<TAB ? 2u : 1u> tg, tu;
+    unit_rows_loop<BITS, RT, NTT, kUnitDepth>(
         wbase, woff, sbt, hidden,
         [&](uint32_t p) { return sorted[gr.first + (p < gr.count ? p : 0u)].token * stride; }, D, unit_lds, acc,
         [&]() {
@@ -553,8 +551,8 @@ __device__ __forceinline__ void unit_down(const ExpertPool& pool, const Pair* __
     const uint32_t nd = D - d_blk < NR ? D - d_blk : NR;
     const uint16_t* ds = reinterpret_cast<const uint16_t*>(blob + o.down_s) + (size_t)d_blk * G;
     const uint16_t* dbv = reinterpret_cast<const uint16_t*>(blob + o.down_b) + (size_t)d_blk * G;
-    TableRegs<TAB ? (RT == 4 ? 2u : 1u) : 1u> td;
-    unit_rows_loop<BITS, RT, NTT, unit_depth<RT>()>(
+    TableRegs<1u> td;
+    unit_rows_loop<BITS, RT, NTT, kUnitDepth>(
         wbase, woff, sbt, act, [&](uint32_t p) { return (gr.first + (p < gr.count ? p : 0u)) * F; }, F, unit_lds, acc,
         [&]() {
             if constexpr (TAB) td.issue(ds, dbv, nd * G, tid);
@@ -718,7 +716,7 @@ static_assert(kUnitThreads == kProjThreads, "the grouped launches run kProjThrea
 
 // TAB: the units' scale/bias tables staged through registers (the host
 // picks these launches for 16-byte aligned scale/bias offsets whose tables
-// fit: d <= 3072 for gate/up, f <= 1024 for down).
+// fit: d <= 4096 for gate/up, f <= 1024 for down).
 template <int BITS, bool TAB = false>
 __device__ __forceinline__ void moe_grouped_gate_up_launch(const ExpertPool& pool, const Pair* __restrict__ sorted,
                                                            const Tile* __restrict__ tiles, uint32_t* __restrict__ n_tiles,
@@ -732,8 +730,8 @@ __device__ __forceinline__ void moe_grouped_gate_up_launch(const ExpertPool& poo
             else unit_gate_up<BITS, 2, 4, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
         },
         [&](const GroupedRows& gr, uint32_t bx) {
-            if (gr.count <= 16u) unit_gate_up<BITS, 4, 1, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
-            else unit_gate_up<BITS, 4, 2, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
+            if (gr.count <= 16u) unit_gate_up<BITS, 2, 1, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
+            else unit_gate_up<BITS, 2, 2, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
         });
 }
 
@@ -749,8 +747,8 @@ __device__ __forceinline__ void moe_grouped_down_launch(const ExpertPool& pool, 
             else unit_down<BITS, 2, 4, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
         },
         [&](const GroupedRows& gr, uint32_t bx) {
-            if (gr.count <= 16u) unit_down<BITS, 4, 1, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
-            else unit_down<BITS, 4, 2, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
+            if (gr.count <= 16u) unit_down<BITS, 2, 1, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
+            else unit_down<BITS, 2, 2, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
         });
 }
 

@@ -329,6 +329,29 @@ def test_grouped_tile_and_stream_split(ctx, stream, bits):
         assert rel < TOL, f"expert {e} ({c} pairs): rel={rel}"
 
 
+@pytest.mark.parametrize("d,f", [(320, 320), (3136, 64), (4096, 64)])
+def test_grouped_stream_unit_edges(ctx, stream, d, f):
+    # pair counts at both sides of the 16-pair sub-tiles and of the stream
+    # cut, an expert without pairs, a partial last row block (320), and the
+    # widest tables of a gate/up unit staged through registers (d <= 4096)
+    k, E = 1, 9
+    counts = [1, 15, 16, 17, 31, 32, 33, 0, 65]
+    T = sum(counts)
+    idx = np.repeat(np.arange(E, dtype=np.uint32), counts).reshape(T, k)
+    w16 = synth.f16_bits(synth.uniform24(synth.seed_key(13, "edges/w"), T * k, 0.1, 0.9)).reshape(T, k)
+    pool_bytes, offs, stride = synth.expert_pool(13, f"edges/{d}", E, d, f)
+    hidden = synth.f16_vector(13, "edges/x", T * d)
+    got, parts, _ = _run_grouped(ctx, stream, pool_bytes, offs, stride, E, idx, w16, hidden, d, T, k, d, f)
+    assert got["status"] == 0 and not np.any(parts == UNWRITTEN)
+    ref = oracle.grouped_route_partials(got["sorted"].astype(oracle.PAIR_DTYPE), hidden, d,
+                                        *_oracle_pool(pool_bytes, offs, stride), k, d, f, T)
+    gp, rp = from_f16_bits(parts).reshape(T, d), from_f16_bits(ref).reshape(T, d)
+    for e, c in enumerate(counts):
+        rows = np.flatnonzero(idx[:, 0] == e)
+        rel = oracle.rel_error(gp[rows], rp[rows]) if c else 0.0
+        assert rel < TOL, f"expert {e} ({c} pairs): rel={rel}"
+
+
 def _repack_misaligned(pool_bytes, offs, stride, E, d, f):
     # the same experts with every scale and bias array at a 2-byte (not
     # 16-byte) aligned offset, weight arrays still 16-byte aligned
