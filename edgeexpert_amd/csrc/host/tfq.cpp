@@ -91,6 +91,9 @@ static std::vector<std::string> kernel_names() {
                           "tfq_q8_block_gated_r2_t2", "tfq_q8_block_gated_r2_t4", "tfq_q8_tile", "tfq_q8_tile_gated"})
         names.push_back(n);
     for (int c = 1; c <= 8; ++c) names.push_back("tfq_router_block_c" + std::to_string(c));
+    for (const char* b : {"2", "3", "4"})
+        for (const char* c : {"1", "2", "3", "4"})
+            names.push_back(std::string("tfq_moe_stream_gate_up_b") + b + "_c" + c);
     for (const char* n : {"tfq_prefill_select", "tfq_moe_group", "tfq_moe_grouped_gate_up", "tfq_moe_grouped_down",
                           "tfq_moe_grouped_gate_up_b2", "tfq_moe_grouped_down_b2", "tfq_moe_grouped_gate_up_b3",
                           "tfq_moe_grouped_down_b3", "tfq_moe_grouped_gate_up_t", "tfq_moe_grouped_down_t",

@@ -72,37 +72,23 @@ __device__ __forceinline__ void transpose_quarters(uint32_t (&t)[4]) {
     t[3] = (uint32_t)d[1];
 }
 
-// RT: 16-row MFMA tiles per wave (1 or 2); X_BF16: X and Y in bf16 (else
-// fp16); rows of X and Y ldx and ldy halves apart; CNT: 128-code tiles per wave, ceil(K / 1024) (a compile-time count,
-// so the loop unrolls and every wait names exactly the tile it needs).
+// The K loop of a block and the sum of its eight K-slices: in wavefront 0 (true
+// is returned there) acc[i] is row tile i in the 16x16 D layout (column lane%16
+// = token, rows 4·(lane/16) + r). wrow, srow, brow: the row lane/4 of each tile;
+// xrow: the token row lane/4. CNT: 128-code tiles per wave, ceil(K / 1024) (a
+// compile-time count, so the loop unrolls and every wait names exactly the tile
+// it needs).
 template <bool X_BF16, int RT, int BITS, int CNT>
-__device__ __forceinline__ void gemm_skinny(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W,
-                                            const uint16_t* __restrict__ S, const uint16_t* __restrict__ B,
-                                            uint16_t* __restrict__ Y, uint32_t M, uint32_t N, uint32_t K,
-                                            uint32_t ldx, uint32_t ldy) {
+__device__ __forceinline__ bool skinny_rows(const uint8_t* const (&wrow)[RT], const uint16_t* const (&srow)[RT],
+                                            const uint16_t* const (&brow)[RT], const uint16_t* __restrict__ xrow,
+                                            uint32_t K, f32x4 (&acc)[RT]) {
     __shared__ f32x4 red[kSkinnyWaves][RT][64];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t r16 = lane & 15u, q = lane >> 4;
     const uint32_t nch = K >> 5;                       // 32-code chunks per row
     const uint32_t G = K >> 6;
-    const uint32_t row_bytes = (K >> 3) * BITS;
-    const uint32_t n0 = blockIdx.x * (16u * RT);
-    const uint32_t t0 = blockIdx.y * kSkinnyTok, t = t0 + r16;
-
-    const uint32_t lrow = lane >> 2, lq = load_quarter(lane), from = operand_source(r16, q);
+    const uint32_t lq = load_quarter(lane), from = operand_source(r16, q);
     const uint32_t ntile = (K + 127u) >> 7;
-    const uint8_t* wrow[RT];
-    const uint16_t* srow[RT];
-    const uint16_t* brow[RT];
-#pragma unroll
-    for (int i = 0; i < RT; ++i) {
-        const uint32_t r = n0 + 16u * i + lrow, rc = r < N ? r : N - 1;    // rows past N: clamped, not stored
-        wrow[i] = W + (size_t)rc * row_bytes;
-        srow[i] = S + (size_t)rc * G;
-        brow[i] = B + (size_t)rc * G;
-    }
-    const uint32_t tl = t0 + lrow;
-    const uint16_t* xrow = X + (size_t)(tl < M ? tl : M - 1) * ldx;      // tokens past M: clamped, not stored
 
     const DequantConsts<BITS> dc = dequant_consts<BITS>();
 
@@ -133,7 +119,6 @@ __device__ __forceinline__ void gemm_skinny(const uint16_t* __restrict__ X, cons
                 sraw[h][i][g] = srow[i][gc];
                 braw[h][i][g] = brow[i][gc];
             }
-    f32x4 acc[RT];
 #pragma unroll
     for (int i = 0; i < RT; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     auto compute = [&](uint32_t m, const SkinnyStage<RT, BITS>& st) {
@@ -191,20 +176,50 @@ __device__ __forceinline__ void gemm_skinny(const uint16_t* __restrict__ X, cons
 #pragma unroll
     for (int i = 0; i < RT; ++i) red[wave][i][lane] = acc[i];
     __syncthreads();
-    if (wave != 0) return;
+    if (wave != 0) return false;
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
-        f32x4 v = red[0][i][lane];
+        acc[i] = red[0][i][lane];
 #pragma unroll
-        for (uint32_t w = 1; w < kSkinnyWaves; ++w) v += red[w][i][lane];
-        // D layout of the 16x16 MFMA: column = lane % 16 (token), rows 4·(lane/16) + r
+        for (uint32_t w = 1; w < kSkinnyWaves; ++w) acc[i] += red[w][i][lane];
+    }
+    return true;
+}
+
+// RT: 16-row MFMA tiles per wave (1 or 2); X_BF16: X and Y in bf16 (else
+// fp16); rows of X and Y ldx and ldy halves apart.
+template <bool X_BF16, int RT, int BITS, int CNT>
+__device__ __forceinline__ void gemm_skinny(const uint16_t* __restrict__ X, const uint8_t* __restrict__ W,
+                                            const uint16_t* __restrict__ S, const uint16_t* __restrict__ B,
+                                            uint16_t* __restrict__ Y, uint32_t M, uint32_t N, uint32_t K,
+                                            uint32_t ldx, uint32_t ldy) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t G = K >> 6, row_bytes = (K >> 3) * BITS;
+    const uint32_t n0 = blockIdx.x * (16u * RT);
+    const uint32_t t0 = blockIdx.y * kSkinnyTok, t = t0 + (lane & 15u), q = lane >> 4;
+    const uint32_t lrow = lane >> 2;
+    const uint8_t* wrow[RT];
+    const uint16_t* srow[RT];
+    const uint16_t* brow[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+        const uint32_t r = n0 + 16u * i + lrow, rc = r < N ? r : N - 1;    // rows past N: clamped, not stored
+        wrow[i] = W + (size_t)rc * row_bytes;
+        srow[i] = S + (size_t)rc * G;
+        brow[i] = B + (size_t)rc * G;
+    }
+    const uint32_t tl = t0 + lrow;
+    const uint16_t* xrow = X + (size_t)(tl < M ? tl : M - 1) * ldx;      // tokens past M: clamped, not stored
+    f32x4 acc[RT];
+    if (!skinny_rows<X_BF16, RT, BITS, CNT>(wrow, srow, brow, xrow, K, acc)) return;
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const uint32_t n = n0 + 16u * i + 4u * q + r;
             if (n < N && t < M)
-                Y[(size_t)t * ldy + n] = X_BF16 ? __builtin_bit_cast(uint16_t, (__bf16)v[r]) : f2h(v[r]);
+                Y[(size_t)t * ldy + n] = X_BF16 ? __builtin_bit_cast(uint16_t, (__bf16)acc[i][r]) : f2h(acc[i][r]);
         }
-    }
 }
 
 }  // namespace tfq

@@ -259,7 +259,7 @@ __device__ __forceinline__ void sfor_while(Fn&& f) {
 // 128-expert block are ~530 gate/up units of them on 512 blocks, two rounds
 // with the second nearly empty, and 704 features leave the last one half
 // empty. With 128 rows: 512 tokens at 4 bits 203.3 -> 195.5 us per call, 33
-// tokens at 3 bits 107.2 -> 101.9. Lane l holds row l%16 of each A operand and the quarter
+// tokens at 3 bits 107.2 -> 102 to 105. Lane l holds row l%16 of each A operand and the quarter
 // q = l/16 of every 128-code k-tile (chunk 4m + q: one 16-byte load at 4 bits;
 // word u feeds k-step u), dequantised from a DEPTH-deep register ring with the
 // scale and bias of an LDS table (one word per row and group). The unit's
@@ -750,6 +750,47 @@ __device__ __forceinline__ void moe_grouped_down_launch(const ExpertPool& pool, 
             if (gr.count <= 16u) unit_down<BITS, 2, 1, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
             else unit_down<BITS, 2, 2, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
         });
+}
+
+// Gate/up + GeGLU of a few pairs per expert as a weight stream (gemm_skinny.hpp):
+// block (16 features, tile), 8 wavefronts over the gate and up rows of those
+// features with K split between them, 16 pairs at a time. A unit's barrier per
+// k-tile is a serial chain that a launch of few units cannot hide; here no
+// wavefront waits for another before the final sum: 2 tokens of top-8 at 2816
+// x 704, 4 bits, 49.1 -> 42.7 us per call, at 3 bits 53.3 -> 45.3. Above about a
+// pair per expert the blocks outnumber the chip several times and read the
+// activations again for every 16 features, and the units are as fast. CNT:
+// ceil(D / 1024).
+template <int BITS, int CNT>
+__device__ __forceinline__ void moe_stream_gate_up(const ExpertPool& pool, const Pair* __restrict__ sorted,
+                                                   const Tile* __restrict__ tiles,
+                                                   const uint32_t* __restrict__ n_tiles,
+                                                   const uint16_t* __restrict__ hidden, uint32_t stride,
+                                                   uint16_t* __restrict__ act, uint32_t D, uint32_t F) {
+    const Tile tile = tiles[blockIdx.y];
+    if (blockIdx.y >= *n_tiles) return;
+    const uint32_t lane = threadIdx.x & 63u, lrow = lane >> 2, r16 = lane & 15u, q = lane >> 4;
+    const uint32_t G = D >> 6, row_bytes = (D >> 3) * BITS;
+    const uint32_t f0 = blockIdx.x * 16u, fl = f0 + lrow, fc = fl < F ? fl : F - 1;   // past F: clamped, not stored
+    const uint8_t* blob = pool.base + (uint64_t)tile.expert * pool.stride;
+    const ExpertOffsets& o = pool.off;
+    const uint8_t* const wrow[2] = {blob + o.gate_w + (size_t)fc * row_bytes, blob + o.up_w + (size_t)fc * row_bytes};
+    const uint16_t* const srow[2] = {reinterpret_cast<const uint16_t*>(blob + o.gate_s) + (size_t)fc * G,
+                                     reinterpret_cast<const uint16_t*>(blob + o.up_s) + (size_t)fc * G};
+    const uint16_t* const brow[2] = {reinterpret_cast<const uint16_t*>(blob + o.gate_b) + (size_t)fc * G,
+                                     reinterpret_cast<const uint16_t*>(blob + o.up_b) + (size_t)fc * G};
+    for (uint32_t p0 = 0; p0 < tile.count; p0 += 16u) {
+        const uint32_t pl = p0 + lrow < tile.count ? p0 + lrow : tile.count - 1;      // past the tile: clamped, not stored
+        const uint16_t* xrow = hidden + (size_t)sorted[tile.start + pl].token * stride;
+        f32x4 acc[2];
+        if (skinny_rows<false, 2, BITS, CNT>(wrow, srow, brow, xrow, D, acc) && p0 + r16 < tile.count) {
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = gelu_tanh(acc[0][r]) * acc[1][r];
+            store_f16x4(act + (size_t)(tile.start + p0 + r16) * F, f0 + 4u * q, F, v);
+        }
+        __syncthreads();             // the sums are read before the next pairs' are written
+    }
 }
 
 // h2[t][d] = fp16(Σ_r fma(w[t][r], partials[(t*k+r)*D + d])) in rank order

@@ -30,3 +30,16 @@ TFQ_GROUPED(_b3, 3, false)
 TFQ_GROUPED(_t, 4, true)
 TFQ_GROUPED(_b2_t, 2, true)
 TFQ_GROUPED(_b3_t, 3, true)
+
+// gate/up of a few pairs per expert: CNT = ceil(d/1024)
+#define TFQ_STREAM_GATE_UP(BITS, CNT)                                                            \
+    extern "C" __global__ __launch_bounds__(kSkinnyThreads) void tfq_moe_stream_gate_up_b##BITS##_c##CNT( \
+        ExpertPool pool, const Pair* sorted, const Tile* tiles, const uint32_t* n_tiles,         \
+        const uint16_t* hidden, uint32_t stride, uint16_t* act, uint32_t D, uint32_t F) {        \
+        moe_stream_gate_up<BITS, CNT>(pool, sorted, tiles, n_tiles, hidden, stride, act, D, F);  \
+    }
+#define TFQ_STREAM_GATE_UP_BITS(BITS) \
+    TFQ_STREAM_GATE_UP(BITS, 1) TFQ_STREAM_GATE_UP(BITS, 2) TFQ_STREAM_GATE_UP(BITS, 3) TFQ_STREAM_GATE_UP(BITS, 4)
+TFQ_STREAM_GATE_UP_BITS(2)
+TFQ_STREAM_GATE_UP_BITS(3)
+TFQ_STREAM_GATE_UP_BITS(4)

@@ -352,6 +352,38 @@ def test_grouped_stream_unit_edges(ctx, stream, d, f):
         assert rel < TOL, f"expert {e} ({c} pairs): rel={rel}"
 
 
+@pytest.mark.parametrize("bits", [4, 3, 2])
+@pytest.mark.parametrize("d", [64, 1088, 2112, 4096])
+def test_grouped_few_pairs_per_expert(ctx, stream, d, bits):
+    # the gate/up weight stream: pair counts at both sides of its 16-pair
+    # passes, experts without pairs, and d at each of its tile counts with a
+    # half-filled last tile (64, 1088, 2112) and at its limit (4096)
+    f, k, E = 64, 1, 112
+    counts = [1, 2, 15, 16, 17, 0, 33] + [0] * (E - 7)
+    T = sum(counts)
+    assert ops.max_tiles(T, k, E) <= E * 3 // 4 + 1
+    idx = np.repeat(np.arange(E, dtype=np.uint32), counts).reshape(T, k)
+    w16 = synth.f16_bits(synth.uniform24(synth.seed_key(14, "few/w"), T * k, 0.1, 0.9)).reshape(T, k)
+    pool_bytes, offs, stride = synth.expert_pool(14, f"few/{d}/b{bits}", E, d, f, bits=bits)
+    hidden = synth.f16_vector(14, "few/x", T * d)
+    got, bufs = _device_group(ctx, stream, idx, w16, T, k, E)
+    assert got["status"] == 0
+    pool = ops.ExpertPool(_dev(pool_bytes), stride, E, offs, weight_bits=bits)
+    act, partials = _dev(np.full(T * f, UNWRITTEN, np.uint16)), _dev(np.full(T * d, UNWRITTEN, np.uint16))
+    ops.PrefillGroupedRoutedMoE(ctx).encode(stream, pool, bufs["sorted"], bufs["tiles"], bufs["n_tiles"],
+                                            ops.max_tiles(T, k, E), _dev(hidden), d, d, f, k, act, partials)
+    stream.sync()
+    parts = partials.download(np.uint16)
+    assert not np.any(act.download(np.uint16) == UNWRITTEN) and not np.any(parts == UNWRITTEN)
+    ref = oracle.grouped_route_partials(got["sorted"].astype(oracle.PAIR_DTYPE), hidden, d,
+                                        *_oracle_pool(pool_bytes, offs, stride), k, d, f, T, bits=bits)
+    gp, rp = from_f16_bits(parts).reshape(T, d), from_f16_bits(ref).reshape(T, d)
+    for e, c in enumerate(counts):
+        rows = np.flatnonzero(idx[:, 0] == e)
+        rel = oracle.rel_error(gp[rows], rp[rows]) if c else 0.0
+        assert rel < TOL, f"expert {e} ({c} pairs): rel={rel}"
+
+
 def _repack_misaligned(pool_bytes, offs, stride, E, d, f):
     # the same experts with every scale and bias array at a 2-byte (not
     # 16-byte) aligned offset, weight arrays still 16-byte aligned
