@@ -106,7 +106,9 @@ struct AttnLds {
 // [num_q_heads][nparts][2].
 // With GB < G every subset block of the new token's part runs the k/v
 // epilogue on the staged raw rows (epi.k_raw / v_raw) and writes the same
-// words into the cache slot; nothing reads that slot from the caches.
+// words into the cache slot. Whatever the clamped loads find in that slot
+// (before or after that write) is replaced: the new token's row by the LDS
+// copy, V rows past it by zeros, scores past it by -inf.
 template <int HD, int G, int GB = G>
 __device__ __forceinline__ void attn_partial(const uint16_t* __restrict__ q, uint16_t* __restrict__ kc,
                                              uint16_t* __restrict__ vc, uint32_t nkv, uint32_t seq_len,
@@ -300,6 +302,13 @@ __device__ __forceinline__ void attn_partial(const uint16_t* __restrict__ q, uin
 #pragma unroll
                 for (int e = 0; e < 8; ++e) o[g][e] *= r;
             }
+        }
+        // V rows past the visible keys: zero, not the clamped load (their p is
+        // 0, but 0 times an infinity or NaN in the last key's slot is NaN)
+        if (!MORE && n < kAttnChunk) {
+#pragma unroll
+            for (uint32_t i = 0; i < KPG; ++i)
+                if (vg * KPG + i >= n) vr[i] = u32x4{0u, 0u, 0u, 0u};
         }
 #pragma unroll
         for (uint32_t i = 0; i < KPG; ++i) {

@@ -155,7 +155,9 @@ def _spec(shape):
                                     attn_scale=shape["scale"])
 
 
-def _layer_case(ctx, stream, shape, E, pos, cap, seed, label, in_place=False, expert_bits=4, shared_bits=4):
+def _layer_case(ctx, stream, shape, E, pos, cap, seed, label, in_place=False, expert_bits=4, shared_bits=4,
+                slot=None):
+    # slot: fp16 bits that fill the caches' row `pos` on entry
     w = synth.decode_layer(seed, label, shape["d"], shape["nq"], shape["nkv"], shape["hd"], E, shape["f"],
                            shape["fs"], expert_bits=expert_bits, shared_bits=shared_bits,
                            v_proj=not shape.get("full", False))
@@ -171,6 +173,9 @@ def _layer_case(ctx, stream, shape, E, pos, cap, seed, label, in_place=False, ex
     ws = DeviceBuffer(ws_bytes)
     ws.fill(0)
     kb, vb, hb = _dev(kc), _dev(vc), _dev(hidden)
+    if slot is not None:
+        for b in (kb, vb):
+            b.upload(np.full(kvd, slot, np.uint16), offset=pos * kvd * 2)
     ob = hb if in_place else _dev(np.full(shape["d"], 0x7E00, np.uint16))
     layer = ops.DecodeLayer(ctx, ops.DecodeLayerWeightsSpec.upload(w), spec)
     layer.encode(stream, hb, ob, kb, vb, pos, ws, ws_bytes)
@@ -318,6 +323,22 @@ CONFIG4_FULL = dict(CONFIG4, nkv=2, hd=512, rotated_pairs=64, theta=1e6, full=Tr
 def test_layer_small_full_attention(ctx, stream, pos):
     got, ref, w, hid = _layer_case(ctx, stream, SMALL_FULL, 8, pos, 160, 10, f"small-full-{pos}")
     _check_layer(got, ref, w, SMALL_FULL, hid, f"small full pos={pos}")
+
+
+@pytest.mark.parametrize("shape,pos", [(SMALL_FULL, 0), (SMALL_FULL, 70), (SMALL_FULL, 16450),
+                                       (dict(SMALL, full=True), 70), (dict(SMALL, hd=256, full=True), 130),
+                                       (dict(SMALL, nq=1, nkv=1, hd=512, full=True), 70), (SMALL, 70)])
+def test_layer_ignores_the_slot_of_the_new_token(ctx, stream, shape, pos):
+    # a cache that was never cleared: the new token's row of both caches holds
+    # NaN or infinity on entry and the last 64-key chunk is ragged, so the
+    # loads past the visible keys are clamped to that row. Every stage's bits
+    # are those of a cleared slot.
+    assert (pos + 1) % 64
+    label = f"slot-{shape['hd']}-{shape['nkv']}-{pos}"
+    runs = [_layer_case(ctx, stream, shape, 8, pos, pos + 1, 17, label, slot=s)[0] for s in (0, 0x7E00, 0x7C00)]
+    for got in runs[1:]:
+        for key in ("attn", "out", "kslot", "vslot", "idx"):
+            assert np.all(np.isfinite(got[key])) and np.array_equal(got[key], runs[0][key]), f"{label}: {key}"
 
 
 @pytest.mark.parametrize("full", [True, False])
