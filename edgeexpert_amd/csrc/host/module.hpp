@@ -63,6 +63,7 @@ public:
         return it == fns_.end() ? nullptr : it->second;
     }
     int device() const { return device_; }
+    uint32_t compute_units() const { return cus_; }
 
     // Blocks of `block` threads and `lds` dynamic LDS bytes that the whole GPU
     // holds resident at once for kernel f (occupancy per CU x CUs); cached

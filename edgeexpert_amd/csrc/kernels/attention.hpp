@@ -13,7 +13,8 @@
 // which is the exact softmax of AttentionRef.apply
 // (V/Reference/Attention/Attention.swift:14-104) regrouped by chunk. When
 // there are more chunks than the GPU holds blocks, a block takes several
-// consecutive chunks as one part, rescaling its (l, O) to the new maximum
+// consecutive chunks as one part (Attention::parts, ops.hpp, shares them out
+// over one or two blocks per CU), rescaling its (l, O) to the new maximum
 // from chunk to chunk: one prologue and one partial row per part, and the
 // next chunk's K rows on their way during the current one's softmax and p·V.
 // 32768 keys per call, one chunk per block and here: 16 query / 2 kv heads of
@@ -97,8 +98,9 @@ struct AttnLds {
     float red[2048 / HD][GB][HD];
 };
 
-// One (part, kv head, query-head subset) block: part blockIdx % nparts, the
-// chunks part·cpb .. of the keys, query heads h·G + z·GB + [0, GB). The
+// One (part, kv head, query-head subset) block: part p = unit % nparts, whose
+// chunks are the `base` (one more in the first `extra` parts) after those of
+// the parts before it, query heads h·G + sub·GB + [0, GB). The
 // subset blocks of one (part, kv head) read the same K and V rows: blocks b
 // and b + 8 of the launch, which the dispatcher hands to the same XCD, so the
 // second finds them in its L2. q: fp16 [num_q_heads][HD] (raw projection when
@@ -114,7 +116,7 @@ __device__ __forceinline__ void attn_partial(const uint16_t* __restrict__ q, uin
                                              uint16_t* __restrict__ vc, uint32_t nkv, uint32_t seq_len,
                                              uint32_t kv_start, float scale, const AttnEpilogue& epi,
                                              float* __restrict__ part_o, float* __restrict__ part_ml,
-                                             uint32_t nparts, uint32_t cpb) {
+                                             uint32_t nparts, uint32_t base, uint32_t extra) {
     static_assert(HD == 128 || HD == 256 || HD == 512, "head_dim 128, 256 or 512");
     static_assert(GB >= 1 && G % GB == 0, "query heads split evenly over blocks");
     constexpr uint32_t CPL = HD / 128;                 // 16-byte pieces per lane per key (q·k)
@@ -141,7 +143,8 @@ __device__ __forceinline__ void attn_partial(const uint16_t* __restrict__ q, uin
     const uint32_t part = unit % nparts, h = unit / nparts;
     const uint32_t qh0 = h * G + sub * GB;                               // first query head of the block
     const uint32_t nchunks = (seq_len - kv_start + kAttnChunk - 1) / kAttnChunk;
-    const uint32_t ch0 = part * cpb, ch1 = ch0 + cpb < nchunks ? ch0 + cpb : nchunks;   // this part's chunks
+    const uint32_t ch0 = part * base + (part < extra ? part : extra);          // this part's chunks
+    const uint32_t ch1 = ch0 + base + (part < extra ? 1u : 0u);
     const size_t row = (size_t)nkv * HD;               // halves between consecutive positions
     const uint16_t* kbase = kc + (size_t)kv_start * row + (size_t)h * HD;
     const uint16_t* vbase = vc + (size_t)kv_start * row + (size_t)h * HD;

@@ -103,15 +103,15 @@ constexpr uint32_t kTailGemvThreads = 1024;
     TFQ_ROUTER_FORM(tfq_router_logits_c_s##SEG##_p##P, (int)kStageCopy, SEG, P)                  \
     TFQ_ROUTER_FORM(tfq_router_logits_pa_s##SEG##_p##P, (int)kStagePostAttn, SEG, P)
 
-// GB: query heads per block (G / GB blocks per (chunk, kv head), blockIdx.z).
+// GB: query heads per block (G / GB blocks per (part, kv head)).
 // two wavefronts per SIMD asked for: 256 registers are the bound, none of them AGPRs
 #define TFQ_ATTN_GB(HD, G, GB)                                                                   \
     extern "C" __global__ __launch_bounds__(kAttnThreads, 2) void tfq_attn_partial_h##HD##_g##G( \
         const uint16_t* q, uint16_t* kc, uint16_t* vc, uint32_t nkv, uint32_t seq_len,           \
         uint32_t kv_start, float scale, AttnEpilogue epi, float* part_o, float* part_ml,         \
-        uint32_t nparts, uint32_t cpb) {                                                          \
+        uint32_t nparts, uint32_t base, uint32_t extra) {                                         \
         attn_partial<HD, G, GB>(q, kc, vc, nkv, seq_len, kv_start, scale, epi, part_o, part_ml,   \
-                                nparts, cpb);                                                     \
+                                nparts, base, extra);                                             \
     }
 #define TFQ_ATTN(HD, G) TFQ_ATTN_GB(HD, G, G)
 

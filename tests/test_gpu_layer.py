@@ -33,9 +33,9 @@ def _dev(a):
 
 # ---------------------------------------------------------------- attention ----
 
-def _run_attention(ctx, stream, q16, k16, v16, hd, nq, nkv, seq, window, scale):
+def _run_attention(ctx, stream, q16, k16, v16, hd, nq, nkv, seq, window, scale, ws=None):
     ws_bytes = ops.Attention.workspace_bytes(hd, nq, seq, window)
-    ws = DeviceBuffer(ws_bytes)
+    ws = ws or DeviceBuffer(ws_bytes)
     out = _dev(np.full(nq * hd, 0x7E00, np.uint16))
     ops.Attention(ctx).encode(stream, _dev(q16), _dev(k16), _dev(v16), out, hd, nq, nkv, seq, ws, ws_bytes,
                               window=window, scale=scale)
@@ -71,14 +71,38 @@ def test_attention_matches_reference(ctx, stream, hd, nq, nkv, seq, window, scal
     assert rel < TOL, f"{tag}: rel={rel}"
 
 
+def _chunks(seq, window):
+    return (min(seq, window or seq) + 63) // 64
+
+
+def _part_workspace(hd, nq, seq, window):
+    """An attention workspace filled with a NaN no kernel stores."""
+    n = ops.Attention.workspace_bytes(hd, nq, seq, window)
+    return _dev(np.full(n // 4, 0x7FFFFFFF, np.uint32))
+
+
+def _parts_written(ws, hd, nq, seq, window):
+    """Parts of each query head: the (m, l) pairs that the partial launch left."""
+    at = (nq * _chunks(seq, window) * hd * 4 + 255) // 256 * 256
+    ml = ws.download(np.uint32, nq * _chunks(seq, window) * 2, offset=at)
+    written = int(np.count_nonzero(ml != 0x7FFFFFFF))
+    assert written % (2 * nq) == 0
+    return written // (2 * nq)
+
+
 @pytest.mark.parametrize("hd,nq,nkv,seq,window", [
-    (512, 16, 2, 8257, 0),       # two chunks per block, the last block with one of one key
-    (512, 16, 2, 24700, 0),      # four chunks, the last block with two, ragged
-    (256, 32, 8, 5000, 0),       # group 4
+    (512, 16, 2, 8257, 0),       # 130 chunks: 44 blocks of at most three per unit
+    (512, 16, 2, 24700, 0),      # 386 chunks, ragged
+    (512, 16, 4, 8300, 0),       # group 4
+    (512, 16, 8, 4200, 0),       # group 2
+    (512, 8, 8, 4200, 0),        # group 1
+    (256, 32, 8, 7000, 0),       # group 4
     (256, 16, 8, 12400, 0),      # group 2
     (256, 16, 8, 30000, 6500),   # a window of more chunks than the GPU holds blocks
-    (128, 16, 8, 13000, 0),
-    (512, 8, 8, 4200, 0),        # group 1
+    (256, 8, 8, 8300, 0),        # group 1
+    (128, 16, 8, 13000, 0),      # group 2
+    (128, 32, 8, 8300, 0),       # group 4
+    (128, 8, 8, 12400, 0),       # group 1
 ])
 @pytest.mark.parametrize("spike", [False, True])
 def test_attention_several_chunks_per_block(ctx, stream, hd, nq, nkv, seq, window, spike):
@@ -94,11 +118,41 @@ def test_attention_several_chunks_per_block(ctx, stream, hd, nq, nkv, seq, windo
         qf = from_f16_bits(q16).reshape(nkv, nq // nkv, hd)
         for j, s in ((seq - 1, 0.02), (seq // 2, 0.05), (seq - (window or seq) + 3, 0.03)):
             k16[j] = synth.f16_bits(qf[:, 0] * s * np.sqrt(hd) / 2)
-    got = _run_attention(ctx, stream, q16, k16, v16, hd, nq, nkv, seq, window, None)
+    ws = _part_workspace(hd, nq, seq, window)
+    got = _run_attention(ctx, stream, q16, k16, v16, hd, nq, nkv, seq, window, None, ws)
+    assert _parts_written(ws, hd, nq, seq, window) < _chunks(seq, window), f"{tag}: one chunk per block"
     ref = oracle.attention(from_f16_bits(q16), from_f16_bits(k16.reshape(-1)), from_f16_bits(v16), hd, nq, nkv, seq,
                            window, None)
     rel = oracle.rel_error(got, ref)
     assert rel < TOL, f"{tag}: rel={rel}"
+
+
+@pytest.mark.parametrize("hd,nq,nkv,seqs", [
+    (256, 16, 8, (4160, 6208, 8192, 8997, 9300, 18528, 32768)), (512, 8, 8, (4160, 8192, 15247)),
+    (512, 16, 2, (8192, 8257, 9965, 24700, 33000)), (128, 16, 8, (11848, 30036))])
+def test_attention_parts_load_the_cus_evenly(ctx, stream, hd, nq, nkv, seqs):
+    # a count of blocks just over a multiple of the CUs leaves some of them with
+    # a block more than the rest and the call waits for those: beyond one chunk
+    # per block there is one block per CU, or two where that leaves the deepest
+    # CU fewer chunks (light chunks: fewer by the measured 5/3)
+    cus = 256
+    units = nkv * (2 if hd == 512 and nq == 8 * nkv else 1)
+    light = hd == 128 or units > nkv
+    for seq in seqs:
+        ws = _part_workspace(hd, nq, seq, 0)
+        kv = DeviceBuffer(seq * nkv * hd * 2)
+        kv.fill(0)
+        ops.Attention(ctx).encode(stream, DeviceBuffer(nq * hd * 2), kv, kv, DeviceBuffer(nq * hd * 2), hd, nq, nkv,
+                                  seq, ws, ws.nbytes)
+        stream.sync()
+        nc, parts = _chunks(seq, 0), _parts_written(ws, hd, nq, seq, 0)
+        if parts == nc:
+            continue
+        per_part, per_cu = -(-nc // parts), -(-parts * units // cus)
+        single = -(-nc // (cus // units))
+        fewer = 5 * per_part < 3 * single if light else 2 * per_part < single
+        assert per_cu == 1 and per_part == single or per_cu == 2 and fewer, \
+            f"{seq} keys: {parts} parts of {per_part} chunks, {per_cu} blocks per CU"
 
 
 def test_attention_is_deterministic(ctx, stream):
