@@ -108,7 +108,7 @@ def bench_c3(ctx, stream, batch_avg_us, bits=4):
     def chunk(i):
         grouping.encode(stream, idx_b, w_b, T, k, E, sorted_p, offsets, counts, tiles, n_tiles, status)
         grouped.encode(stream, pool, sorted_p, tiles, n_tiles, mt, hid.ptr((i % n_hidden) * T * D * 2), D, D, F,
-                       k, act, partials)
+                       k, act, partials, pairs=n)
         grouped.encode_reduce_token_major(stream, partials, w_b, h2, T, k, D)
 
     us = batch_avg_us(chunk, 8, reps_=3)

@@ -154,6 +154,8 @@ SIGNATURES = {
                              C.POINTER(C.c_int64), C.POINTER(C.c_int64)],
     "tfq_moe_grouped": [_P, _P, C.POINTER(ExpertPoolDesc), _P, _P, _P, _U32, _P, _U32, _U32, _U32,
                         _U32, _P, _P],
+    "tfq_moe_grouped_pairs": [_P, _P, C.POINTER(ExpertPoolDesc), _P, _P, _P, _U32, _U32, _P, _U32, _U32,
+                              _U32, _U32, _P, _P],
     "tfq_moe_combine": [_P, _P, _P, _P, _P, _U32, _U32, _U32],
     "tfq_moe_prefill_workspace_bytes": [_U32, _U32, _U32, _U32, _U32],
     "tfq_moe_prefill": [_P, _P, C.POINTER(RouterDesc), C.POINTER(ExpertPoolDesc), _P, _U32, _U32,

@@ -995,7 +995,7 @@ public:
 
     int encode(void* stream, const tfq_expert_pool& pool, const tfq_pair* sorted,
                const tfq_tile* tiles, uint32_t* n_tiles, uint32_t max_tiles,
-               const uint16_t* hidden, uint32_t stride, uint32_t d, uint32_t f, uint32_t k,
+               uint32_t n_pairs, const uint16_t* hidden, uint32_t stride, uint32_t d, uint32_t f, uint32_t k,
                uint16_t* act, uint16_t* partials) const {
         int rc = check_expert_pool(pool, d, f);
         if (rc) return rc;
@@ -1045,12 +1045,14 @@ public:
         };
         GroupedLaunch g1{max_tiles, (f + 63) / 64, (f + 63) / 64};
         uint32_t grid1 = 0, grid2 = 0;
-        // fewer pairs than 3/4 of the experts (the bound is then one tile per
-        // pair and one more), so that most active experts have one or two:
-        // gate/up as a weight stream. Per call at 128 experts, top-8, 4 bits,
-        // with it and with the units: 2 tokens 42.7 and 49.1 us, 8 tokens 64.7
-        // and 68.1, 12 tokens 73.9 and 74.4, 16 tokens 78.5 and 76.4
-        if (d <= 4096 && max_tiles <= pool.num_experts * 3u / 4u + 1u) {
+        // at most 3/4 as many pairs as experts, so that most active experts
+        // have one or two: gate/up as a weight stream. Only where the caller
+        // states the pairs: a tile bound says nothing of them (64 tiles may be
+        // 64 pairs or 8192), and the stream reads a tile's weights again for
+        // every 16 of its pairs. Per call at 128 experts, top-8, 4 bits, with
+        // it and with the units: 2 tokens 42.7 and 49.1 us, 8 tokens 64.7 and
+        // 68.1, 12 tokens 73.9 and 74.4, 16 tokens 78.5 and 76.4
+        if (d <= 4096 && n_pairs && n_pairs <= pool.num_experts * 3u / 4u) {
             char name[48];
             std::snprintf(name, sizeof(name), "tfq_moe_stream_gate_up_b%u_c%u", bits, (d + 1023) / 1024);
             void* a1[] = {&kp, &sorted, &tiles, &n_tiles, &hidden, &stride, &act, &d, &f};

@@ -550,9 +550,17 @@ int tfq_moe_grouped(tfq_ctx* ctx, void* stream, const tfq_expert_pool* pool, con
                     const tfq_tile* tiles, uint32_t* n_tiles, uint32_t max_tiles,
                     const uint16_t* hidden, uint32_t hidden_stride, uint32_t d, uint32_t f,
                     uint32_t top_k, uint16_t* act_scratch, uint16_t* route_partials) {
+    return tfq_moe_grouped_pairs(ctx, stream, pool, sorted, tiles, n_tiles, max_tiles, 0, hidden, hidden_stride, d,
+                                 f, top_k, act_scratch, route_partials);
+}
+
+int tfq_moe_grouped_pairs(tfq_ctx* ctx, void* stream, const tfq_expert_pool* pool, const tfq_pair* sorted,
+                          const tfq_tile* tiles, uint32_t* n_tiles, uint32_t max_tiles, uint32_t n_pairs,
+                          const uint16_t* hidden, uint32_t hidden_stride, uint32_t d, uint32_t f, uint32_t top_k,
+                          uint16_t* act_scratch, uint16_t* route_partials) {
     TFQ_REQUIRE_CTX(ctx);
     if (!pool) return fail(TFQ_E_INVAL, "null pool");
-    return ctx->grouped->encode(stream, *pool, sorted, tiles, n_tiles, max_tiles, hidden,
+    return ctx->grouped->encode(stream, *pool, sorted, tiles, n_tiles, max_tiles, n_pairs, hidden,
                                 hidden_stride, d, f, top_k, act_scratch, route_partials);
 }
 
@@ -624,7 +632,7 @@ int tfq_moe_prefill(tfq_ctx* ctx, void* stream, const tfq_router* router, const 
     if (rc) return rc;
     auto* partials = reinterpret_cast<uint16_t*>(ws + L.partials);
     rc = ctx->grouped->encode(stream, *pool, sorted, tiles, n_tiles, TFQ_MOE_MAX_TILES(T, top_k, E),
-                              hidden, hidden_stride, d, f, top_k,
+                              T * top_k, hidden, hidden_stride, d, f, top_k,
                               reinterpret_cast<uint16_t*>(ws + L.act), partials);
     if (rc) return rc;
     return ctx->grouped->encode_reduce_token_major(stream, partials, out_weights, h2, T, top_k, d);

@@ -505,12 +505,13 @@ class PrefillGroupedRoutedMoE:
         self.ctx = context
 
     def encode(self, stream, pool: "ExpertPool", sorted_pairs, tiles, n_tiles, max_tiles_, hidden,
-               hidden_stride, d, f, top_k, act_scratch, route_partials):
+               hidden_stride, d, f, top_k, act_scratch, route_partials, pairs=0):
+        """pairs: how many were grouped (query_count·top_k), for the kernels of few pairs; 0: not known."""
         p = pool.desc()
-        check(lib().tfq_moe_grouped(self.ctx.handle, _s(stream), C.byref(p), _addr(sorted_pairs),
-                                    _addr(tiles), _addr(n_tiles), max_tiles_, _addr(hidden),
-                                    hidden_stride, d, f, top_k, _addr(act_scratch),
-                                    _addr(route_partials)), "PrefillGroupedRoutedMoE.encode")
+        check(lib().tfq_moe_grouped_pairs(self.ctx.handle, _s(stream), C.byref(p), _addr(sorted_pairs),
+                                          _addr(tiles), _addr(n_tiles), max_tiles_, pairs, _addr(hidden),
+                                          hidden_stride, d, f, top_k, _addr(act_scratch),
+                                          _addr(route_partials)), "PrefillGroupedRoutedMoE.encode")
 
     def encode_reduce_token_major(self, stream, route_partials, route_weights, h2, query_count,
                                   top_k, d):

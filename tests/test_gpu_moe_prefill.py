@@ -397,7 +397,7 @@ def test_grouped_few_pairs_per_expert(ctx, stream, d, bits):
     f, k, E = 64, 1, 112
     counts = [1, 2, 15, 16, 17, 0, 33] + [0] * (E - 7)
     T = sum(counts)
-    assert ops.max_tiles(T, k, E) <= E * 3 // 4 + 1
+    assert T * k <= E * 3 // 4
     idx = np.repeat(np.arange(E, dtype=np.uint32), counts).reshape(T, k)
     w16 = synth.f16_bits(synth.uniform24(synth.seed_key(14, "few/w"), T * k, 0.1, 0.9)).reshape(T, k)
     pool_bytes, offs, stride = synth.expert_pool(14, f"few/{d}/b{bits}", E, d, f, bits=bits)
@@ -407,13 +407,37 @@ def test_grouped_few_pairs_per_expert(ctx, stream, d, bits):
     pool = ops.ExpertPool(_dev(pool_bytes), stride, E, offs, weight_bits=bits)
     act, partials = _dev(np.full(T * f, UNWRITTEN, np.uint16)), _dev(np.full(T * d, UNWRITTEN, np.uint16))
     ops.PrefillGroupedRoutedMoE(ctx).encode(stream, pool, bufs["sorted"], bufs["tiles"], bufs["n_tiles"],
-                                            ops.max_tiles(T, k, E), _dev(hidden), d, d, f, k, act, partials)
+                                            ops.max_tiles(T, k, E), _dev(hidden), d, d, f, k, act, partials,
+                                            pairs=T * k)
     stream.sync()
     a, parts = act.download(np.uint16), partials.download(np.uint16)
     assert not np.any(a == UNWRITTEN) and not np.any(parts == UNWRITTEN)
     _check_grouped_fp16(from_f16_bits(a).astype(np.float64).reshape(T, f),
                         from_f16_bits(parts).astype(np.float64).reshape(T, d), got["sorted"].astype(oracle.PAIR_DTYPE),
                         from_f16_bits(hidden).astype(np.float64).reshape(T, d), pool_bytes, offs, stride, d, f, k, bits)
+
+
+def test_grouped_kernel_does_not_depend_on_the_tile_bound(ctx, stream):
+    # full tiles with a launch bound that is the real tile count: no fewer
+    # pairs for it, so the same kernels and bits as with the loose bound
+    d, f, k, E = 704, 64, 1, 96
+    T = 40 * 100
+    idx = np.repeat(np.arange(40, dtype=np.uint32), 100).reshape(T, k)
+    w16 = np.full((T, k), 0x3C00, np.uint16)
+    pool_bytes, offs, stride = synth.expert_pool(15, "tight", E, d, f)
+    hidden = _dev(synth.f16_vector(15, "tight/x", T * d))
+    pool = ops.ExpertPool(_dev(pool_bytes), stride, E, offs)
+    got, bufs = _device_group(ctx, stream, idx, w16, T, k, E)
+    assert got["n_tiles"] == 40 <= E * 3 // 4
+    out = []
+    for bound in (ops.max_tiles(T, k, E), got["n_tiles"]):
+        act, partials = _dev(np.full(T * f, UNWRITTEN, np.uint16)), _dev(np.full(T * d, UNWRITTEN, np.uint16))
+        ops.PrefillGroupedRoutedMoE(ctx).encode(stream, pool, bufs["sorted"], bufs["tiles"], bufs["n_tiles"], bound,
+                                                hidden, d, d, f, k, act, partials)
+        stream.sync()
+        out.append((act.download(np.uint16), partials.download(np.uint16)))
+    assert not np.any(out[0][1] == UNWRITTEN)
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
 
 
 def _repack_misaligned(pool_bytes, offs, stride, E, d, f):
