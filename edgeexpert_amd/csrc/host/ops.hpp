@@ -1011,11 +1011,10 @@ public:
             return fail(TFQ_E_UNSUPPORTED, "max_tiles=%u exceeds %u (8192 pairs over 256 experts)", max_tiles,
                         kGroupMaxTiles);
         ExpertPool kp = kernel_pool(pool);
-        // one launch per projection over the work list of the tiles: tiles of
-        // at most 32 pairs as stream units, larger ones as 64-pair halves on
-        // wide units (64 features / 128 outputs per unit either way); the
-        // grid is the blocks the GPU holds resident, at most the units the
-        // tile bound allows
+        // one launch per projection over the work list of the tiles, whole or
+        // (more than 32 pairs) as 64-pair halves, times blocks of 64 features
+        // / 128 outputs; the grid is the blocks the GPU holds resident, at
+        // most the units the tile bound allows
         const uint32_t bits = pool_bits(pool);
         // the _t launches stage each unit's scale/bias table through
         // registers: 16-byte aligned scale/bias arrays (base and stride are)
@@ -1039,11 +1038,11 @@ public:
             hipFunction_t fn = m_.get(name);
             if (!fn) return fail(TFQ_E_NOT_LOADED, "kernel %s is not in the code object", name);
             const uint32_t p = m_.resident_blocks(fn, kUnitThreads, lds);
-            const uint32_t units = 2u * max_tiles * std::max(g.wx, g.sx);
+            const uint32_t units = 2u * max_tiles * g.row_blocks;
             grid = std::min(p, units);
             return TFQ_OK;
         };
-        GroupedLaunch g1{max_tiles, (f + 63) / 64, (f + 63) / 64};
+        GroupedLaunch g1{max_tiles, (f + 63) / 64};
         uint32_t grid1 = 0, grid2 = 0;
         // at most 3/4 as many pairs as experts, so that most active experts
         // have one or two: gate/up as a weight stream. Only where the caller
@@ -1064,7 +1063,7 @@ public:
             rc = launch2(m_, gu, grid1, 1, kUnitThreads, lds_for(d), stream, a1);
         }
         if (rc) return rc;
-        GroupedLaunch g2{max_tiles, (d + 127) / 128, (d + 127) / 128};
+        GroupedLaunch g2{max_tiles, (d + 127) / 128};
         rc = grid_for(dn, g2, lds_for(f), grid2);
         if (rc) return rc;
         void* a2[] = {&kp, &sorted, &tiles, &n_tiles, &act, &partials, &d, &f, &k, &g2};

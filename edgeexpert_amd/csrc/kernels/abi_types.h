@@ -146,12 +146,11 @@ struct Tile {
 };
 
 // Shape of one grouped launch (moe_prefill.hpp): the tile list's bound and
-// the row blocks per entry of the two roles; the grid is the resident
-// blocks, which walk the work list.
+// the row blocks per entry; the grid is the resident blocks, which walk the
+// work list.
 struct GroupedLaunch {
     uint32_t max_tiles;
-    uint32_t wx;      // row blocks of the wide role
-    uint32_t sx;      // row blocks of the stream
+    uint32_t row_blocks;
 };
 
 }  // namespace tfq

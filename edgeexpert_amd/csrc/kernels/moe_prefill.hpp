@@ -28,9 +28,9 @@ constexpr uint32_t kGroupSegments = 8;         // chunk segments of the per-expe
 // status codes (the PrefillMoEGroupingError cases the device can detect)
 constexpr uint32_t kGroupOk = 0;
 constexpr uint32_t kGroupExpertOutOfRange = 8;
-// grouping tiles of at most kGroupStreamMax pairs run as stream units, larger
-// ones as wide units (see the grouped MoE units below)
-constexpr uint32_t kGroupStreamMax = 32;
+// grouping tiles of at most kGroupWholeMax pairs run as one unit per row block,
+// larger ones as halves (see the grouped MoE units below)
+constexpr uint32_t kGroupWholeMax = 32;
 
 // threadIdx.x as an opaque value: the work units of a persistent launch read
 // it through this, so the compiler rederives each unit's lane addresses
@@ -219,7 +219,7 @@ __device__ __forceinline__ void moe_group(const uint32_t* __restrict__ idx, cons
 // Rows of one work unit's pairs: a run of the sorted pairs of one expert.
 struct GroupedRows {
     uint32_t first;   // index of the first pair in the sorted pairs
-    uint32_t count;   // pairs (1..64 on the wide role, 1..32 on the stream)
+    uint32_t count;   // pairs (1..64)
     uint32_t expert;
 };
 
@@ -248,19 +248,18 @@ __device__ __forceinline__ void sfor_while(Fn&& f) {
 // ------------------------------------------------------ grouped MoE units ----
 //
 // The grouped projections run per unit: the pairs of one grouping tile (a
-// 64-pair half of a tile of more than kGroupStreamMax pairs, or a whole
-// smaller tile) times a block of weight rows. Each of the four wavefronts owns
-// RT 16-row A operands of v_mfma_f32_16x16x32_f16 and the whole K loop; the
-// pairs are NTT 16-pair B operands: RT 2, 128 rows per unit (gate/up: 64
-// features, gate and up rows; down: 128 outputs) for wide units (tiles of more
-// than 32 pairs, NTT 2 or 4) and stream units (the others, NTT 1 or 2) alike.
-// Stream units of 256 rows (RT 4) spread an activation k-tile over twice the
-// rows but are too few to share out evenly over the blocks: 33 tokens of a
-// 128-expert block are ~530 gate/up units of them on 512 blocks, two rounds
-// with the second nearly empty, and 704 features leave the last one half
-// empty. With 128 rows: 512 tokens at 4 bits 203.3 -> 195.5 us per call, 33
-// tokens at 3 bits 107.2 -> 102 to 105. Lane l holds row l%16 of each A operand and the quarter
-// q = l/16 of every 128-code k-tile (chunk 4m + q: one 16-byte load at 4 bits;
+// 64-pair half of a tile of more than kGroupWholeMax pairs, or a whole
+// smaller tile) times a block of 128 weight rows (gate/up: the gate and up rows
+// of 64 features; down: 128 outputs). Each of the four wavefronts owns RT = 2
+// 16-row A operands of v_mfma_f32_16x16x32_f16 and the whole K loop; the pairs
+// are NTT = 1, 2 or 4 16-pair B operands. Units of 256 rows (RT 4) spread an
+// activation k-tile over twice the rows but are too few to share out evenly
+// over the blocks: 33 tokens of a 128-expert block are ~530 gate/up units of
+// them on 512 blocks, two rounds with the second nearly empty, and 704
+// features leave the last one half empty. With 128 rows: 512 tokens at 4 bits
+// 203.3 -> 195.5 us per call, 33 tokens at 3 bits 107.2 -> 104.6. Lane l holds
+// row l%16 of each A operand and the quarter q = l/16 of every 128-code k-tile
+// (chunk 4m + q: one 16-byte load at 4 bits;
 // word u feeds k-step u), dequantised from a DEPTH-deep register ring with the
 // scale and bias of an LDS table (one word per row and group). The unit's
 // activations are staged per k-tile into a double-buffered LDS tile
@@ -271,20 +270,18 @@ __device__ __forceinline__ void sfor_while(Fn&& f) {
 // zero weights) against activations staged from column 0 (finite), so they
 // add nothing. Weights are dequantised as everywhere else (fp16(q·s + b),
 // one rounding).
-constexpr uint32_t kGroupWidePairs = 64;          // pairs of a wide unit (a half tile)
+constexpr uint32_t kGroupHalfPairs = 64;          // pairs of a half tile
+constexpr int kUnitRowTiles = 2;                  // RT
 constexpr uint32_t kUnitStride = 128 + 8;         // halves per LDS activation row
 constexpr uint32_t kUnitThreads = 256;            // four wavefronts
 
 // LDS of a unit: two activation buffers of 16·NTT rows, then the scale/bias
-// table of its 64·RT weight rows.
+// table of its 64·RT weight rows (K/64 words each).
 constexpr uint32_t unit_xbuf(int NTT) { return 16u * (uint32_t)NTT * kUnitStride; }   // halves
-constexpr uint32_t unit_lds_bytes(int RT, int NTT, uint32_t K) {
-    return 2u * unit_xbuf(NTT) * 2u + 4u * 64u * (uint32_t)RT * (K / 64u);
-}
 
 // A unit's scale/bias table staged through registers: the `count` scale and
-// bias words of its rows (16-byte aligned, count % 8 == 0, count <=
-// 8·U·kUnitThreads) loaded by issue() with unconditional, clamped loads
+// bias words of its rows (K/64 per row; 16-byte aligned, count % 8 == 0, count
+// <= 8·U·kUnitThreads, which the host checks) loaded by issue() with unconditional, clamped loads
 // before the unit's weight and activation loads, and written to LDS as
 // (scale | bias << 16) words by store() once they arrive, so the wait for
 // them covers nothing issued after them (copy_sb_to_lds loads and stores in
@@ -321,11 +318,6 @@ struct TableRegs {
         }
     }
 };
-
-// Table words per 16-byte register piece of TableRegs: a unit of `rows`
-// weight rows over K/64 groups fits U pieces per thread when rows·K/64 <=
-// 8·U·kUnitThreads.
-constexpr uint32_t table_regs_fit(uint32_t rows, uint32_t K, uint32_t U) { return rows * (K / 64u) <= 8u * U * kUnitThreads; }
 
 // Global addresses are a block-uniform base (scalar registers) plus a 32-bit
 // per-lane offset, the form that costs one vector register. acc[i][j]: row
@@ -444,14 +436,15 @@ constexpr int kUnitDepth = 3;                // k-tiles of weights in the ring
 // tiles 0..RT/2-1 and its up rows as row tiles RT/2..RT-1, so each lane holds
 // gate and up of the same (pair, feature). LDS table rows 0..NF-1: gate
 // scales/biases, NF..2NF-1: up. TAB: the table staged through registers
-// (TableRegs; 16-byte aligned scale/bias rows, table_regs_fit), else copied
+// (TableRegs; 16-byte aligned scale/bias rows that fit it), else copied
 // by copy_sb_to_lds.
-template <int BITS, int RT, int NTT, bool TAB>
+template <int BITS, int NTT, bool TAB>
 __device__ __forceinline__ void unit_gate_up(const ExpertPool& pool, const Pair* __restrict__ sorted,
                                              const GroupedRows& gr, const uint16_t* __restrict__ hidden,
                                              uint32_t stride, uint16_t* __restrict__ act, uint32_t D, uint32_t F,
                                              uint32_t bx) {
     extern __shared__ __attribute__((aligned(16))) _Float16 unit_lds[];
+    constexpr int RT = kUnitRowTiles;
     constexpr uint32_t NF = 32u * RT, HT = RT / 2;
     const uint32_t tid = unit_tid(), lane = tid & 63u, wave = tid >> 6;
     const uint32_t r16 = lane & 15u, q = lane >> 4;
@@ -516,12 +509,13 @@ __device__ __forceinline__ void unit_gate_up(const ExpertPool& pool, const Pair*
 
 // Down projection of one unit over 64·RT outputs of D (row block bx): wave
 // w takes rows d_blk + 16·RT·w + (0..16·RT-1). TAB as in unit_gate_up.
-template <int BITS, int RT, int NTT, bool TAB>
+template <int BITS, int NTT, bool TAB>
 __device__ __forceinline__ void unit_down(const ExpertPool& pool, const Pair* __restrict__ sorted,
                                           const GroupedRows& gr, const uint16_t* __restrict__ act,
                                           uint16_t* __restrict__ partials, uint32_t D, uint32_t F, uint32_t k,
                                           uint32_t bx) {
     extern __shared__ __attribute__((aligned(16))) _Float16 unit_lds[];
+    constexpr int RT = kUnitRowTiles;
     constexpr uint32_t NR = 64u * RT;
     const uint32_t tid = unit_tid(), lane = tid & 63u, wave = tid >> 6;
     const uint32_t r16 = lane & 15u, q = lane >> 4;
@@ -581,31 +575,26 @@ __device__ __forceinline__ void unit_down(const ExpertPool& pool, const Pair* __
 // A grouped launch runs a grid of resident blocks (P = gridDim.x) over a work
 // list that every block derives from the device tile list, so no block of
 // the launch finds itself without work. A unit is (entry, row block): an
-// entry is one 64-pair half of a tile of more than kGroupStreamMax pairs
-// (wide role, wx row blocks) or one smaller tile (stream, sx row blocks).
-// Entries come in four classes, dearest first: wide halves of more than 32
-// pairs (NTT 4), the other wide halves (NTT 2), stream tiles of 17..32 pairs
-// (NTT 2), then of at most 16 (NTT 1); tile order within a class, and the
+// entry is one 64-pair half of a tile of more than kGroupWholeMax pairs or one
+// smaller tile. Entries come in four classes, dearest first: halves of more
+// than 32 pairs (NTT 4), the other halves, whole tiles of 17..32 pairs (NTT
+// 2), then of at most 16 (NTT 1); tile order within a class, and the
 // row blocks of an entry as consecutive units. Block b runs unit b first and
 // then takes units P, P+1, ... in the order blocks ask for them (a counter in
 // the grouping state, asked one unit ahead), so the dearest units start
 // first and the cheap ones fill the gaps at the end. The last block to leave
 // zeroes the counters for the next launch.
 constexpr uint32_t kGroupMaxTiles = kGroupMaxPairs / kGemmBM + kGroupMaxExperts;   // bound of TFQ_MOE_MAX_TILES
-static_assert(kGemmBM == 2 * kGroupWidePairs, "a grouping tile is two wide halves");
+static_assert(kGemmBM == 2 * kGroupHalfPairs, "a grouping tile is two halves");
 constexpr uint32_t kGroupMaxEntries = 2u * kGroupMaxTiles;
 constexpr uint32_t kGroupNextUnit = 1, kGroupBlocksDone = 2;   // counter words of the grouping state
 
-struct UnitPlan {
-    uint32_t n_wide;      // wide entries (the first two classes)
-    uint32_t n_entries;   // all entries
-};
-
 // Wavefront 0 writes the entries ({first pair, expert | count << 16}) of the
-// first min(n_tiles[0], max_tiles) tiles into ent; ends with a barrier.
-__device__ __forceinline__ UnitPlan plan_units(const Tile* __restrict__ tiles, const uint32_t* __restrict__ n_tiles,
+// first min(n_tiles[0], max_tiles) tiles into ent; ends with a barrier and
+// returns how many there are.
+__device__ __forceinline__ uint32_t plan_units(const Tile* __restrict__ tiles, const uint32_t* __restrict__ n_tiles,
                                                uint32_t max_tiles, uint2* ent) {
-    __shared__ uint32_t plan_tot[2];
+    __shared__ uint32_t n_entries;
     constexpr uint32_t C = kGroupMaxTiles / 64u;          // tiles per lane
     static_assert(kGroupMaxTiles % 64u == 0, "whole wavefront passes");
     if (threadIdx.x < 64u) {
@@ -650,14 +639,14 @@ __device__ __forceinline__ UnitPlan plan_units(const Tile* __restrict__ tiles, c
 #pragma unroll
         for (uint32_t c = 0; c < C; ++c) {
             const Tile t = tl[c];
-            if (t.count > kGroupStreamMax) {
+            if (t.count > kGroupWholeMax) {
                 const uint32_t p0 = pre_w[c] & 0xFFFFu;
-                const uint32_t c0 = t.count < kGroupWidePairs ? t.count : kGroupWidePairs;
+                const uint32_t c0 = t.count < kGroupHalfPairs ? t.count : kGroupHalfPairs;
                 ent[p0] = make_uint2(t.start, t.expert | (c0 << 16));
-                if (t.count > kGroupWidePairs) {
-                    const uint32_t left = t.count - kGroupWidePairs;
+                if (t.count > kGroupHalfPairs) {
+                    const uint32_t left = t.count - kGroupHalfPairs;
                     ent[left > 32u ? p0 + 1u : n0 + (pre_w[c] >> 16)] =
-                        make_uint2(t.start + kGroupWidePairs, t.expert | (left << 16));
+                        make_uint2(t.start + kGroupHalfPairs, t.expert | (left << 16));
                 }
             } else if (t.count > 16u) {
                 ent[n0 + n1 + (pre_s[c] & 0xFFFFu)] = make_uint2(t.start, t.expert | (t.count << 16));
@@ -665,40 +654,29 @@ __device__ __forceinline__ UnitPlan plan_units(const Tile* __restrict__ tiles, c
                 ent[n0 + n1 + n2 + (pre_s[c] >> 16)] = make_uint2(t.start, t.expert | (t.count << 16));
             }
         }
-        if (lane == 0) {
-            plan_tot[0] = n0 + n1;
-            plan_tot[1] = n0 + n1 + n2 + n3;
-        }
+        if (lane == 0) n_entries = n0 + n1 + n2 + n3;
     }
     __syncthreads();
-    return {plan_tot[0], plan_tot[1]};
+    return n_entries;
 }
 
-// The unit loop of one grouped launch: wide(rows, bx) / stream(rows, bx) run
-// one unit each (block-uniform calls). Every unit starts after a barrier, so
-// it may reuse the dynamic LDS of the one before. state: the grouping state
-// (tile count, then the counters).
-template <typename Wide, typename Stream>
+// The unit loop of one grouped launch: unit(rows, bx) runs one (block-uniform
+// calls). Every unit starts after a barrier, so it may reuse the dynamic LDS of
+// the one before. state: the grouping state (tile count, then the counters).
+template <typename Unit>
 __device__ __forceinline__ void run_units(const Tile* __restrict__ tiles, uint32_t* __restrict__ state,
-                                          GroupedLaunch gl, Wide wide, Stream stream) {
+                                          GroupedLaunch gl, Unit unit) {
     __shared__ uint2 ent[kGroupMaxEntries];
     __shared__ uint32_t next_unit;
-    const UnitPlan pl = plan_units(tiles, state, gl.max_tiles, ent);
+    const uint32_t n_units = plan_units(tiles, state, gl.max_tiles, ent) * gl.row_blocks;
     const uint32_t P = gridDim.x, tid = threadIdx.x;
-    const uint32_t n_wu = pl.n_wide * gl.wx, n_units = n_wu + (pl.n_entries - pl.n_wide) * gl.sx;
     uint32_t u = blockIdx.x;
     while (u < n_units) {
         // the next unit's number, asked for now and read after this unit
         uint32_t ask = 0;
         if (tid == 0) ask = atomicAdd(state + kGroupNextUnit, 1u);
-        if (u < n_wu) {
-            const uint2 e = ent[u / gl.wx];
-            wide(GroupedRows{e.x, e.y >> 16, e.y & 0xFFFFu}, u % gl.wx);
-        } else {
-            const uint32_t v = u - n_wu;
-            const uint2 e = ent[pl.n_wide + v / gl.sx];
-            stream(GroupedRows{e.x, e.y >> 16, e.y & 0xFFFFu}, v % gl.sx);
-        }
+        const uint2 e = ent[u / gl.row_blocks];
+        unit(GroupedRows{e.x, e.y >> 16, e.y & 0xFFFFu}, u % gl.row_blocks);
         if (tid == 0) next_unit = ask + P;
         __syncthreads();
         u = next_unit;
@@ -723,16 +701,11 @@ __device__ __forceinline__ void moe_grouped_gate_up_launch(const ExpertPool& poo
                                                            const uint16_t* __restrict__ hidden, uint32_t stride,
                                                            uint16_t* __restrict__ act, uint32_t D, uint32_t F,
                                                            GroupedLaunch gl) {
-    run_units(
-        tiles, n_tiles, gl,
-        [&](const GroupedRows& gr, uint32_t bx) {
-            if (gr.count <= 32u) unit_gate_up<BITS, 2, 2, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
-            else unit_gate_up<BITS, 2, 4, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
-        },
-        [&](const GroupedRows& gr, uint32_t bx) {
-            if (gr.count <= 16u) unit_gate_up<BITS, 2, 1, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
-            else unit_gate_up<BITS, 2, 2, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
-        });
+    run_units(tiles, n_tiles, gl, [&](const GroupedRows& gr, uint32_t bx) {
+        if (gr.count <= 16u) unit_gate_up<BITS, 1, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
+        else if (gr.count <= 32u) unit_gate_up<BITS, 2, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
+        else unit_gate_up<BITS, 4, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
+    });
 }
 
 template <int BITS, bool TAB = false>
@@ -740,16 +713,11 @@ __device__ __forceinline__ void moe_grouped_down_launch(const ExpertPool& pool, 
                                                         const Tile* __restrict__ tiles, uint32_t* __restrict__ n_tiles,
                                                         const uint16_t* __restrict__ act, uint16_t* __restrict__ partials,
                                                         uint32_t D, uint32_t F, uint32_t k, GroupedLaunch gl) {
-    run_units(
-        tiles, n_tiles, gl,
-        [&](const GroupedRows& gr, uint32_t bx) {
-            if (gr.count <= 32u) unit_down<BITS, 2, 2, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
-            else unit_down<BITS, 2, 4, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
-        },
-        [&](const GroupedRows& gr, uint32_t bx) {
-            if (gr.count <= 16u) unit_down<BITS, 2, 1, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
-            else unit_down<BITS, 2, 2, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
-        });
+    run_units(tiles, n_tiles, gl, [&](const GroupedRows& gr, uint32_t bx) {
+        if (gr.count <= 16u) unit_down<BITS, 1, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
+        else if (gr.count <= 32u) unit_down<BITS, 2, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
+        else unit_down<BITS, 4, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
+    });
 }
 
 // Gate/up + GeGLU of a few pairs per expert as a weight stream (gemm_skinny.hpp):

@@ -136,8 +136,8 @@ def test_grouped_down_one_hot_is_bit_exact(ctx, stream, bits):
     # e^(-2z) underflows) and each down partial of a pair of token t is the
     # expert's dequantised down weight of column t: fp16(q·s + b), one
     # rounding. Routing: rank 0 -> expert 0 (128 pairs: two 64-pair halves on
-    # wide units), rank 1 -> experts 1..15 (8-9 pairs: stream units), rank 2 ->
-    # experts 16..18 (42-43 pairs: one partly filled wide half); expert 19 idle.
+    # their own units), rank 1 -> experts 1..15 (8-9 pairs: whole tiles), rank 2 ->
+    # experts 16..18 (42-43 pairs: one partly filled half); expert 19 idle.
     T, k, E, D, F = 128, 3, 20, 256, 128
     offs, stride = synth.expert_layout(D, F, align=256, bits=bits)
     pool = np.zeros(E * stride, np.uint8)

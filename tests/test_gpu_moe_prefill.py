@@ -282,7 +282,7 @@ def test_grouped_moe_baseline_config3_sampled(ctx, stream):
     rel = oracle.rel_error(from_f16_bits(h2).reshape(T, d)[toks], ref_h2[toks])
     assert rel < TOL, f"h2 rel={rel}"
     # and the first and last pair of every active expert: every grouping tile,
-    # both halves of the wide ones and every unit class is checked
+    # both halves of the larger ones and every unit class is checked
     srt = got["sorted"]
     ends = sorted({i for e in np.unique(srt["expert"])
                    for i in (int(np.flatnonzero(srt["expert"] == e)[0]), int(np.flatnonzero(srt["expert"] == e)[-1]))})
