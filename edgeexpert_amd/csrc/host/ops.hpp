@@ -1107,28 +1107,28 @@ public:
         return ((size_t)nq * nc * head_dim * 4 + 255) / 256 * 256 + ((size_t)nq * nc * 2 * 4 + 255) / 256 * 256;
     }
 
-    // Parts that the `chunks` chunks of one unit (kv head, query-head subset)
-    // are shared out to, a block per part and unit. One chunk per part while
-    // the GPU holds all blocks at once (`room`). Else one or two blocks per CU:
-    // a part takes c = ceil(chunks / parts that fit) chunks, and the choice is
-    // the one with fewer chunks on a CU (c at one block, 2c at two), one block
-    // on a tie, since two share its bandwidth. Where a chunk is little work for
-    // its memory round trips (`light`: head_dim 128; the half groups of
-    // head_dim 512, which share K and V) two blocks cost 5/3 of one. A third
-    // block per CU never paid: the counts between do not spread evenly.
-    // us per call with ceil(blocks / room) chunks per block, one chunk per
-    // block, and here, 16 query / 8 kv heads of 256: 8192 keys 22.8, 20.5,
-    // 17.4; 8997 keys 25.5, 21.7, 17.0; 18528 keys 36.0, 40.8, 29.1; 8 / 8 heads
-    // of 512, 7519 keys 25.4, 30.0, 25.2; 16 / 2 of 512, 9965 keys 22.1, 21.5, 20.5.
-    static uint32_t parts(uint32_t chunks, uint32_t units, uint32_t room, uint32_t cus, bool light) {
-        if ((uint64_t)chunks * units <= room) return chunks;
+    // Chunks per part for the `chunks` chunks of one unit (kv head, query-head
+    // subset), a block per part and unit. One chunk while the GPU holds all
+    // blocks at once (`room`), at three per CU at most, whatever more of them
+    // the registers allow. Else one or two blocks per CU: a part takes c =
+    // ceil(chunks / parts that fit) chunks, and the choice is the one with
+    // fewer chunks on a CU (c at one block, 2c at two), one block on a tie,
+    // since two share its bandwidth. Where a chunk is little work for its
+    // memory round trips (`light`: head_dim 128; the half groups of head_dim
+    // 512, which share K and V) two blocks cost 5/3 of one. More blocks do not
+    // spread evenly over the CUs, and the call waits for the fullest. us per
+    // call with ceil(blocks / room) chunks per block, one chunk per block, and
+    // here, 16 query / 8 kv heads of 256: 8192 keys 22.8, 20.5, 17.4; 8997 keys
+    // 25.5, 21.7, 17.0; 18528 keys 36.0, 40.8, 29.1; 8 / 8 heads of 512, 7519
+    // keys 25.4, 30.0, 25.2; 16 / 2 of 512, 9965 keys 22.1, 21.5, 20.5.
+    static uint32_t chunks_per_part(uint32_t chunks, uint32_t units, uint32_t room, uint32_t cus, bool light) {
+        if ((uint64_t)chunks * units <= std::min(room, 3 * cus)) return 1;
         auto per_part = [&](uint32_t blocks) {
             const uint32_t fit = std::max(1u, blocks / units);
             return (chunks + fit - 1) / fit;
         };
         const uint32_t c1 = per_part(cus), c2 = per_part(std::max(cus, std::min(2 * cus, room)));
-        const uint32_t c = c1 * (light ? 3u : 1u) <= c2 * (light ? 5u : 2u) ? c1 : c2;
-        return (chunks + c - 1) / c;
+        return c1 * (light ? 3u : 1u) <= c2 * (light ? 5u : 2u) ? c1 : c2;
     }
 
     // q: fp16 [nq][hd]; caches fp16 [capacity][nkv][hd]; out fp16 [nq][hd].
@@ -1180,11 +1180,10 @@ public:
         std::snprintf(name, sizeof(name), "tfq_attn_partial_h%u_g%u", hd, G);
         hipFunction_t pf = m_.get(name);
         if (!pf) return fail(TFQ_E_NOT_LOADED, "kernel %s is not in the code object", name);
-        uint32_t nparts = parts(nc, nkv * nsub, m_.resident_blocks(pf, 256, 0), m_.compute_units(),
-                                hd == 128 || nsub > 1);
-        uint32_t base = nc / nparts, extra = nc % nparts;
-        void* a1[] = {&q, &k_cache, &v_cache, &nkv, &seq_len, &ks, &scale, &e, &part_o, &part_ml,
-                      &nparts, &base, &extra};
+        uint32_t cpb = chunks_per_part(nc, nkv * nsub, m_.resident_blocks(pf, 256, 0), m_.compute_units(),
+                                       hd == 128 || nsub > 1);
+        uint32_t nparts = (nc + cpb - 1) / cpb;
+        void* a1[] = {&q, &k_cache, &v_cache, &nkv, &seq_len, &ks, &scale, &e, &part_o, &part_ml, &nparts, &cpb};
         int rc = hip_check(hipModuleLaunchKernel(pf, nparts * nkv * nsub, 1, 1, 256, 1, 1, 0, (hipStream_t)stream, a1,
                                                  nullptr),
                            name);

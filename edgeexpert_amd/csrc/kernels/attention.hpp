@@ -13,7 +13,7 @@
 // which is the exact softmax of AttentionRef.apply
 // (V/Reference/Attention/Attention.swift:14-104) regrouped by chunk. When
 // there are more chunks than the GPU holds blocks, a block takes several
-// consecutive chunks as one part (Attention::parts, ops.hpp, shares them out
+// consecutive chunks as one part (Attention::chunks_per_part, ops.hpp, shares them out
 // over one or two blocks per CU), rescaling its (l, O) to the new maximum
 // from chunk to chunk: one prologue and one partial row per part, and the
 // next chunk's K rows on their way during the current one's softmax and p·V.
@@ -98,9 +98,8 @@ struct AttnLds {
     float red[2048 / HD][GB][HD];
 };
 
-// One (part, kv head, query-head subset) block: part p = unit % nparts, whose
-// chunks are the `base` (one more in the first `extra` parts) after those of
-// the parts before it, query heads h·G + sub·GB + [0, GB). The
+// One (part, kv head, query-head subset) block: part unit % nparts, the chunks
+// part·cpb .. of the keys, query heads h·G + sub·GB + [0, GB). The
 // subset blocks of one (part, kv head) read the same K and V rows: blocks b
 // and b + 8 of the launch, which the dispatcher hands to the same XCD, so the
 // second finds them in its L2. q: fp16 [num_q_heads][HD] (raw projection when
@@ -109,14 +108,14 @@ struct AttnLds {
 // With GB < G every subset block of the new token's part runs the k/v
 // epilogue on the staged raw rows (epi.k_raw / v_raw) and writes the same
 // words into the cache slot. Whatever the clamped loads find in that slot
-// (before or after that write) is replaced: the new token's row by the LDS
-// copy, V rows past it by zeros, scores past it by -inf.
+// (before or after that write) is replaced: the new token's row, and V rows
+// past it, by the LDS copy, scores past it by -inf.
 template <int HD, int G, int GB = G>
 __device__ __forceinline__ void attn_partial(const uint16_t* __restrict__ q, uint16_t* __restrict__ kc,
                                              uint16_t* __restrict__ vc, uint32_t nkv, uint32_t seq_len,
                                              uint32_t kv_start, float scale, const AttnEpilogue& epi,
                                              float* __restrict__ part_o, float* __restrict__ part_ml,
-                                             uint32_t nparts, uint32_t base, uint32_t extra) {
+                                             uint32_t nparts, uint32_t cpb) {
     static_assert(HD == 128 || HD == 256 || HD == 512, "head_dim 128, 256 or 512");
     static_assert(GB >= 1 && G % GB == 0, "query heads split evenly over blocks");
     constexpr uint32_t CPL = HD / 128;                 // 16-byte pieces per lane per key (q·k)
@@ -143,8 +142,7 @@ __device__ __forceinline__ void attn_partial(const uint16_t* __restrict__ q, uin
     const uint32_t part = unit % nparts, h = unit / nparts;
     const uint32_t qh0 = h * G + sub * GB;                               // first query head of the block
     const uint32_t nchunks = (seq_len - kv_start + kAttnChunk - 1) / kAttnChunk;
-    const uint32_t ch0 = part * base + (part < extra ? part : extra);          // this part's chunks
-    const uint32_t ch1 = ch0 + base + (part < extra ? 1u : 0u);
+    const uint32_t ch0 = part * cpb, ch1 = ch0 + cpb < nchunks ? ch0 + cpb : nchunks;   // this part's chunks
     const size_t row = (size_t)nkv * HD;               // halves between consecutive positions
     const uint16_t* kbase = kc + (size_t)kv_start * row + (size_t)h * HD;
     const uint16_t* vbase = vc + (size_t)kv_start * row + (size_t)h * HD;
@@ -306,18 +304,14 @@ __device__ __forceinline__ void attn_partial(const uint16_t* __restrict__ q, uin
                 for (int e = 0; e < 8; ++e) o[g][e] *= r;
             }
         }
-        // V rows past the visible keys: zero, not the clamped load (their p is
-        // 0, but 0 times an infinity or NaN in the last key's slot is NaN)
-        if (!MORE && n < kAttnChunk) {
-#pragma unroll
-            for (uint32_t i = 0; i < KPG; ++i)
-                if (vg * KPG + i >= n) vr[i] = u32x4{0u, 0u, 0u, 0u};
-        }
 #pragma unroll
         for (uint32_t i = 0; i < KPG; ++i) {
             const uint32_t j = vg * KPG + i;
             u32x4 vv = vr[i];
-            if (own_pos && kv_start + k0 + j == pos) vv = *reinterpret_cast<const u32x4*>(&L.vp[8u * vl]);
+            // the new token's row, and in its place every row past it: those
+            // loads were clamped to its slot, which may hold anything (their p
+            // is 0, but 0 times a NaN or an infinity there would be NaN)
+            if (own_pos && kv_start + k0 + j >= pos) vv = *reinterpret_cast<const u32x4*>(&L.vp[8u * vl]);
             const h8 v8 = __builtin_bit_cast(h8, vv);
 #pragma unroll
             for (int g = 0; g < GB; ++g) {

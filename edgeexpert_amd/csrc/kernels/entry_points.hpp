@@ -109,9 +109,9 @@ constexpr uint32_t kTailGemvThreads = 1024;
     extern "C" __global__ __launch_bounds__(kAttnThreads, 2) void tfq_attn_partial_h##HD##_g##G( \
         const uint16_t* q, uint16_t* kc, uint16_t* vc, uint32_t nkv, uint32_t seq_len,           \
         uint32_t kv_start, float scale, AttnEpilogue epi, float* part_o, float* part_ml,         \
-        uint32_t nparts, uint32_t base, uint32_t extra) {                                         \
+        uint32_t nparts, uint32_t cpb) {                                                          \
         attn_partial<HD, G, GB>(q, kc, vc, nkv, seq_len, kv_start, scale, epi, part_o, part_ml,   \
-                                nparts, base, extra);                                             \
+                                nparts, cpb);                                                     \
     }
 #define TFQ_ATTN(HD, G) TFQ_ATTN_GB(HD, G, G)
 
