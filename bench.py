@@ -598,7 +598,7 @@ def bench_gemm_policy(ctx, stream, batch_avg_us):
     """The prefill GEMM's kernel choice by token count (config 2's weights,
     N 8192 x K 2816, bf16): the library's choice at token counts on both
     sides of its crossover (112 tokens at this N), and both kernels forced at
-    the two counts next to it."""
+    the last count on the stream and at 128."""
     from edgeexpert_amd import ops, synth
     from edgeexpert_amd._lib import DTYPE_BF16, GEMM_PATH_SKINNY32, GEMM_PATH_TILE
     from edgeexpert_amd.runtime import DeviceBuffer
@@ -615,12 +615,12 @@ def bench_gemm_policy(ctx, stream, batch_avg_us):
     def run(m, path):
         return batch_avg_us(lambda i: q.encode(stream, *bufs[i % copies], X, Y, m, N, Kd, DTYPE_BF16, path=path),
                             32, reps_=3)
-    for m in (1, 16, 64, 80, 96, 128, 512):
+    for m in (1, 16, 64, 96, 112, 128, 512):
         us = run(m, None)
         out["auto"][str(m)] = {"us": round(us, 2), "tflops": round(2.0 * m * N * Kd / (us * 1e-6) / 1e12, 1),
                                "weight_gbs": round(wbytes / (us * 1e-6) / 1e9, 1),
                                "kernel": "gemv" if m == 1 else "skinny" if m <= 112 else "tile"}
-    for m in (64, 96):
+    for m in (112, 128):
         out["forced"][str(m)] = {"skinny32_us": round(run(m, GEMM_PATH_SKINNY32), 2),
                                  "tile_us": round(run(m, GEMM_PATH_TILE), 2)}
     # few tokens: the decode GEMV once per token against the weight stream

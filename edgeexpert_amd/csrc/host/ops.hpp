@@ -28,9 +28,12 @@ constexpr uint32_t kUnitStride = 128 + 8;       // halves per LDS activation row
 constexpr uint32_t kGroupMaxTiles = 8192 / 128 + 256;  // tiles the device planner takes (moe_prefill.hpp)
 // int8 rows over a block of tokens (gemm_q8.hpp)
 constexpr uint32_t kQ8RowTokens = 4;            // most tokens that run the decode kernels once per token
-constexpr uint32_t kQ8FewTokens = 64;           // most tokens on the K-split form (down at 96 tokens: 12.4 against
-                                                // 14.7 us for the tile, gate/up 18.6 against 19.6; at 192 30 against
-                                                // 14.8 and 32 against 20)
+// most tokens on the K-split form. Both launches of a call, K-split and tile, at
+// 2816 x 2112: 48 tokens 27.1 and 35.8 us, 64: 30.6 and 36.0, 72: 36.0 and 35.5,
+// 96: 42.8 and 35.8; at 4096 x 4096 64 tokens 46.3 and 56.9, 65: 62.0 and 56.2.
+// Matrices of few row blocks would take it further (2816 x 704: 24.2 and 26.8 us
+// at 65 tokens, even at 150; 640 x 320 11.7 and 13.2)
+constexpr uint32_t kQ8FewTokens = 64;
 constexpr uint32_t kQ8BlockThreads = 512;       // threads of the K-split form
 constexpr uint32_t kQ8TileThreads = 256;        // threads, tokens and weight rows of the tile
 constexpr uint32_t kQ8TileTok = 64;

@@ -52,7 +52,7 @@ M_SWEEP = [1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 24, 31, 32, 33, 47, 48, 63, 64, 6
 
 @pytest.mark.parametrize("n", [2048, 8192])
 def test_auto_path_over_token_counts(ctx, stream, n):
-    # M = 1 ... past the crossover on both sides, every output row of every token
+    # M = 1 ... past the crossover at N 8192, every output row of every token
     k = 2816
     W, S, B = synth.int4_matrix(21, f"policy/w{n}", n, k)
     X = synth.f16_vector(21, "policy/x", max(M_SWEEP) * k).reshape(-1, k)
@@ -62,6 +62,22 @@ def test_auto_path_over_token_counts(ctx, stream, n):
         print(f"[policy] n={n} m={t}", flush=True)
         y = _gemm(ctx, stream, bufs, t, n, k, DTYPE_F16)
         _check(y, ref_all[:t], DTYPE_F16, f"n={n} m={t}")
+
+
+@pytest.mark.parametrize("n,last", [(2048, 448), (2816, 320), (8192, 112)])
+def test_auto_path_next_to_the_crossover(ctx, stream, n, last):
+    # the weight stream up to `last` tokens, the tile from the next one on: the
+    # bits of the forced path, and the first and last tokens against the oracle
+    k = 2816
+    W, S, B = synth.int4_matrix(25, f"cross/w{n}", n, k)
+    X = synth.f16_vector(25, "cross/x", (last + 1) * k).reshape(-1, k)
+    bufs = (_dev(W), _dev(S), _dev(B), _dev(X))
+    for t, path in ((last, GEMM_PATH_SKINNY32), (last + 1, GEMM_PATH_TILE)):
+        y = _gemm(ctx, stream, bufs, t, n, k, DTYPE_F16)
+        assert np.array_equal(y, _gemm(ctx, stream, bufs, t, n, k, DTYPE_F16, path=path)), f"n={n} t={t}"
+        for rows in ((0, 2), (t - 2, t)):
+            ref = oracle.gemm_int4(W, S, B, from_f16_bits(X[:t]), rows=rows)
+            _check(y[rows[0]:rows[1]], ref[rows[0]:rows[1]], DTYPE_F16, f"n={n} t={t}")
 
 
 @pytest.mark.parametrize("n", [2048, 2816, 4096, 8192])

@@ -150,10 +150,11 @@ def test_prefill_shared_expert_block_matches_rows(ctx, stream, bits, xs):
             assert oracle.rel_error(got[r], one) < TOL, f"row {r}: block vs row"
 
 
-@pytest.mark.parametrize("bits,rows", [(8, 24), (4, 24), (4, 80)])
+@pytest.mark.parametrize("bits,rows", [(8, 24), (4, 24), (4, 80), (4, 450)])
 def test_prefill_shared_expert_config4_shape(ctx, stream, bits, rows):
-    # the C4 shared expert (d 2816, f 2112) over a block of rows; int4 at 24 rows
-    # takes the few-token GEMM, at 80 rows the MFMA tile
+    # the C4 shared expert (d 2816, f 2112) over a block of rows; int4 at 24 and
+    # 80 rows takes the few-token GEMM, at 450 rows the MFMA tile (above 432
+    # rows at 2112 outputs, 320 at 2816), each with padded rows of x and y
     d, f = 2816, 2112
     print(f"[pshared] bits={bits} rows={rows}", flush=True)
     mats = _synthetic(3, f"pshared{bits}", d, f, bits)
