@@ -778,11 +778,24 @@ inline uint32_t skinny_max_tokens(uint32_t n, uint32_t k) {
     return t < 16 ? 16 : t;
 }
 
+// Most tokens on the loads for a handful of tokens (gemm_skinny.hpp
+// skinny_loads): handing over operands loaded in memory order costs them 0.2 to
+// 1 us, and reading more tokens in operand order costs more. us in memory order
+// and in these, bf16: 2048 x 2816, 8 tokens 5.6 and 5.3, 12 5.7 and 5.8 (at 3 bits
+// 10 tokens 5.7 and 5.3, 12 5.8 and 5.6); 32-row blocks, 8192 x 2816 (one per CU),
+// 12 tokens 8.8 and 8.3, 16384 x 2816, 6 tokens 11.9 and 11.5 (fp16 11.3 and
+// 11.3), 8 fp16 11.4 and 11.8;
+// 2816 x 4096, 6 tokens 7.1 and 6.9, 8 7.2 and 7.1 (fp16 6.7 and 6.9).
+inline uint32_t skinny_few_tokens(uint32_t bits, uint32_t cnt, uint32_t rt, uint32_t blocks) {
+    if (cnt > 3 || blocks > 256) return 6;
+    return cnt == 3 && (rt == 2 || bits == 3) ? 12 : 8;
+}
+
 inline GemmPlan plan_gemm(uint32_t t, uint32_t n, uint32_t k) {
-    // one token: the decode GEMV (N 2048: 3.9 against 4.2 us for the weight
-    // stream, N 8192: 5.8 against 6.3 us, cold weights); from two tokens on
+    // one token: the decode GEMV (N 2048: 4.0 against 4.5 us for the weight
+    // stream, N 8192: 6.1 against 6.8 us, cold weights); from two tokens on
     // the stream reads the weights once for up to 16 tokens and wins (N 8192,
-    // two tokens: 6.3 against 11.2 us for two GEMVs)
+    // two tokens: 6.5 against 11.7 us for two GEMVs)
     if (t == 1) return {TFQ_GEMM_PATH_GEMV};
     if (t > skinny_max_tokens(n, k)) return {TFQ_GEMM_PATH_TILE};
     // 16 rows per wave while that gives at most one block per CU (2816 x 4096,
@@ -837,11 +850,13 @@ public:
             return TFQ_OK;
         }
         if (path == TFQ_GEMM_PATH_SKINNY || path == TFQ_GEMM_PATH_SKINNY32) {
-            const uint32_t rt = path == TFQ_GEMM_PATH_SKINNY32 ? 2 : 1;
+            const uint32_t rt = path == TFQ_GEMM_PATH_SKINNY32 ? 2 : 1, cnt = (k + 1023) / 1024;
+            const uint32_t gx = (n + 16 * rt - 1) / (16 * rt);
+            const bool few = t <= skinny_few_tokens(bits, cnt, rt, gx);
             char sname[64];
-            std::snprintf(sname, sizeof(sname), "tfq_gemm_skinny_q%u_%s_r%u_c%u", bits,
-                          dtype == TFQ_DTYPE_BF16 ? "bf16" : "f16", rt, (k + 1023) / 1024);
-            const uint32_t gx = (n + 16 * rt - 1) / (16 * rt), gy = (t + kSkinnyTok - 1) / kSkinnyTok;
+            std::snprintf(sname, sizeof(sname), "tfq_gemm_skinny_q%u_%s_r%u_c%u%s", bits,
+                          dtype == TFQ_DTYPE_BF16 ? "bf16" : "f16", rt, cnt, few ? "_few" : "");
+            const uint32_t gy = (t + kSkinnyTok - 1) / kSkinnyTok;
             void* args[] = {&x, &weights, &scales, &biases, &y, &t, &n, &k, &ldx, &ldy};
             return launch2(m_, sname, gx, gy, kSkinnyThreads, 0, stream, args);
         }

@@ -85,8 +85,9 @@ static std::vector<std::string> kernel_names() {
         for (const char* dt : {"f16", "bf16"})
             for (const char* rt : {"r1", "r2"})
                 for (int c = 1; c <= 8; ++c)
-                    names.push_back(std::string("tfq_gemm_skinny_") + b + "_" + dt + "_" + rt + "_c" +
-                                    std::to_string(c));
+                    for (const char* few : {"", "_few"})
+                        names.push_back(std::string("tfq_gemm_skinny_") + b + "_" + dt + "_" + rt + "_c" +
+                                        std::to_string(c) + few);
     for (const char* n : {"tfq_q8_block_r1_t1", "tfq_q8_block_r1_t2", "tfq_q8_block_r1_t4", "tfq_q8_block_gated_r2_t1",
                           "tfq_q8_block_gated_r2_t2", "tfq_q8_block_gated_r2_t4", "tfq_q8_tile", "tfq_q8_tile_gated"})
         names.push_back(n);

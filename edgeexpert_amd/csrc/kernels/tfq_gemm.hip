@@ -16,15 +16,17 @@ TFQ_GEMM(q3, 3, f16, false)
 TFQ_GEMM(q3, 3, bf16, true)
 
 // Few-token form (gemm_skinny.hpp): RT 16-row MFMA tiles per wave, C = ceil(K/1024)
-// 128-code tiles per wave.
-#define TFQ_SKINNY(TAG, BITS, DT, X_BF16, RT, C)                                                 \
-    extern "C" __global__ __launch_bounds__(kSkinnyThreads) void                                  \
-        tfq_gemm_skinny_##TAG##_##DT##_r##RT##_c##C(const uint16_t* X, const uint8_t* W,          \
-                                                    const uint16_t* S, const uint16_t* B,         \
-                                                    uint16_t* Y, uint32_t M, uint32_t N,          \
-                                                    uint32_t K, uint32_t ldx, uint32_t ldy) {     \
-        gemm_skinny<X_BF16, RT, BITS, C>(X, W, S, B, Y, M, N, K, ldx, ldy);                       \
+// 128-code tiles per wave; _few: the loads for a handful of tokens.
+#define TFQ_SKINNY_FORM(NAME, BITS, X_BF16, RT, C, LOADS)                                        \
+    extern "C" __global__ __launch_bounds__(kSkinnyThreads) void NAME(                            \
+        const uint16_t* X, const uint8_t* W, const uint16_t* S, const uint16_t* B, uint16_t* Y,   \
+        uint32_t M, uint32_t N, uint32_t K, uint32_t ldx, uint32_t ldy) {                         \
+        gemm_skinny<X_BF16, RT, BITS, C, LOADS>(X, W, S, B, Y, M, N, K, ldx, ldy);                \
     }
+#define TFQ_SKINNY(TAG, BITS, DT, X_BF16, RT, C)                                                 \
+    TFQ_SKINNY_FORM(tfq_gemm_skinny_##TAG##_##DT##_r##RT##_c##C, BITS, X_BF16, RT, C, kLoadsMemory) \
+    TFQ_SKINNY_FORM(tfq_gemm_skinny_##TAG##_##DT##_r##RT##_c##C##_few, BITS, X_BF16, RT, C,       \
+                    skinny_loads(C))
 #define TFQ_SKINNY_C(TAG, BITS, DT, X_BF16, RT)                                                  \
     TFQ_SKINNY(TAG, BITS, DT, X_BF16, RT, 1) TFQ_SKINNY(TAG, BITS, DT, X_BF16, RT, 2)              \
     TFQ_SKINNY(TAG, BITS, DT, X_BF16, RT, 3) TFQ_SKINNY(TAG, BITS, DT, X_BF16, RT, 4)              \

@@ -64,6 +64,28 @@ def test_auto_path_over_token_counts(ctx, stream, n):
         _check(y, ref_all[:t], DTYPE_F16, f"n={n} m={t}")
 
 
+@pytest.mark.parametrize("bits", [4, 3])
+@pytest.mark.parametrize("k", [64, 704, 1088, 2048, 3072, 3136, 7360])
+def test_handful_of_tokens(ctx, stream, k, bits):
+    # the loads in operand order (both operands up to 3072 inputs, x beyond) at
+    # both sides of their token limits, with half-filled last tiles and waves
+    # without tiles, 16 and 32 rows per wave, a partial row block; an infinity
+    # in one token's last column leaves the bits of the other tokens
+    n, T = 50, 13
+    W, S, B = synth.affine_matrix(26, f"few/w{k}", n, k, bits)
+    X = synth.f16_vector(26, "few/x", T * k).reshape(T, k)
+    bad = X.copy()
+    bad[1, k - 1] = 0x7C00
+    ref = oracle.gemm_int4(W, S, B, from_f16_bits(X), bits=bits)
+    bufs = [(_dev(W), _dev(S), _dev(B), _dev(x)) for x in (X, bad)]
+    for path in (GEMM_PATH_SKINNY, GEMM_PATH_SKINNY32):
+        for t in (2, 3, 6, 7, 8, 9, 12, 13):
+            y, z = (_gemm(ctx, stream, b, t, n, k, DTYPE_F16, bits=bits, path=path) for b in bufs)
+            _check(y, ref[:t], DTYPE_F16, f"k={k} t={t} path={path}")
+            rows = [i for i in range(t) if i != 1]
+            assert np.array_equal(y[rows], z[rows]) and not np.any(np.isfinite(z[1])), f"k={k} t={t} path={path}"
+
+
 @pytest.mark.parametrize("n,last", [(2048, 448), (2816, 320), (8192, 112)])
 def test_auto_path_next_to_the_crossover(ctx, stream, n, last):
     # the weight stream up to `last` tokens, the tile from the next one on: the
