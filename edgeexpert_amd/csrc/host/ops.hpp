@@ -1046,9 +1046,18 @@ public:
         char gu[48], dn[48];
         const char* bsuf = bits == 2 ? "_b2" : bits == 3 ? "_b3" : "";
         std::snprintf(gu, sizeof(gu), "tfq_moe_grouped_gate_up%s%s", bsuf, tab_gu ? "_t" : "");
-        std::snprintf(dn, sizeof(dn), "tfq_moe_grouped_down%s%s", bsuf, tab_dn ? "_t" : "");
+        // _w: tiles of at most 32 pairs as units of 256 outputs of down, where a
+        // unit's few k-tiles leave its start (table, ring, first activations) a
+        // large part of it and the units are enough for two blocks per CU. us of
+        // both launches with 128 and 256 outputs, 128 experts, top-8: 2816 x 512
+        // at 4 bits, 16 tokens 57.4 and 54.8, 128 92.3 and 86.8, 512 134.7 and
+        // 132.6; 2816 x 704 at 2 bits, 24 tokens 78.9 and 71.3, 512 153.1 and 151.2,
+        // at 4 bits 33 tokens 82.7 and 86.3; 2 tokens 1024 x 512 16.0 and 18.3
+        const bool wide = f <= (bits == 2 ? 704u : 512u) && max_tiles * ((d + 255) / 256) >= 2 * m_.compute_units();
+        std::snprintf(dn, sizeof(dn), "tfq_moe_grouped_down%s%s%s", bsuf, tab_dn ? "_t" : "", wide ? "_w" : "");
         // dynamic LDS: the largest unit (two activation buffers of 64 pairs,
-        // then the table of 128 rows of K/64 words)
+        // then the table of 128 rows of K/64 words; of 32 pairs and 256 rows
+        // up to 704 codes it takes less)
         auto lds_for = [](uint32_t K) {
             return 2u * 64u * kUnitStride * 2u + 4u * 128u * (K / 64u);
         };
@@ -1056,11 +1065,11 @@ public:
             hipFunction_t fn = m_.get(name);
             if (!fn) return fail(TFQ_E_NOT_LOADED, "kernel %s is not in the code object", name);
             const uint32_t p = m_.resident_blocks(fn, kUnitThreads, lds);
-            const uint32_t units = 2u * max_tiles * g.row_blocks;
+            const uint32_t units = 2u * max_tiles * std::max(g.half_blocks, g.small_blocks);
             grid = std::min(p, units);
             return TFQ_OK;
         };
-        GroupedLaunch g1{max_tiles, (f + 63) / 64};
+        GroupedLaunch g1{max_tiles, (f + 63) / 64, (f + 63) / 64};
         uint32_t grid1 = 0, grid2 = 0;
         // at most 3/4 as many pairs as experts, so that most active experts
         // have one or two: gate/up as a weight stream. Only where the caller
@@ -1081,7 +1090,7 @@ public:
             rc = launch2(m_, gu, grid1, 1, kUnitThreads, lds_for(d), stream, a1);
         }
         if (rc) return rc;
-        GroupedLaunch g2{max_tiles, (d + 127) / 128};
+        GroupedLaunch g2{max_tiles, (d + 127) / 128, wide ? (d + 255) / 256 : (d + 127) / 128};
         rc = grid_for(dn, g2, lds_for(f), grid2);
         if (rc) return rc;
         void* a2[] = {&kp, &sorted, &tiles, &n_tiles, &act, &partials, &d, &f, &k, &g2};

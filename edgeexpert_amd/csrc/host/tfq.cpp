@@ -95,12 +95,14 @@ static std::vector<std::string> kernel_names() {
     for (const char* b : {"2", "3", "4"})
         for (const char* c : {"1", "2", "3", "4"})
             names.push_back(std::string("tfq_moe_stream_gate_up_b") + b + "_c" + c);
-    for (const char* n : {"tfq_prefill_select", "tfq_moe_group", "tfq_moe_grouped_gate_up", "tfq_moe_grouped_down",
-                          "tfq_moe_grouped_gate_up_b2", "tfq_moe_grouped_down_b2", "tfq_moe_grouped_gate_up_b3",
-                          "tfq_moe_grouped_down_b3", "tfq_moe_grouped_gate_up_t", "tfq_moe_grouped_down_t",
-                          "tfq_moe_grouped_gate_up_b2_t", "tfq_moe_grouped_down_b2_t", "tfq_moe_grouped_gate_up_b3_t",
-                          "tfq_moe_grouped_down_b3_t", "tfq_moe_combine", "tfq_moe_combine_x8"})
+    for (const char* n : {"tfq_prefill_select", "tfq_moe_group", "tfq_moe_combine", "tfq_moe_combine_x8"})
         names.push_back(n);
+    for (const char* b : {"", "_b2", "_b3"})
+        for (const char* t : {"", "_t"})
+            for (const char* n : {"gate_up", "down", "down_w"}) {
+                const std::string k = n;
+                names.push_back("tfq_moe_grouped_" + k.substr(0, k.find("_w")) + b + t + (k == "down_w" ? "_w" : ""));
+            }
     names.push_back("tfq_convert_bf16_f16");
     for (const char* hd : {"128", "256", "512"}) {
         for (const char* g : {"1", "2", "4"})

@@ -146,11 +146,12 @@ struct Tile {
 };
 
 // Shape of one grouped launch (moe_prefill.hpp): the tile list's bound and
-// the row blocks per entry; the grid is the resident blocks, which walk the
-// work list.
+// the row blocks per half tile and per whole small tile; the grid is the
+// resident blocks, which walk the work list.
 struct GroupedLaunch {
     uint32_t max_tiles;
-    uint32_t row_blocks;
+    uint32_t half_blocks;
+    uint32_t small_blocks;
 };
 
 }  // namespace tfq

@@ -250,13 +250,14 @@ __device__ __forceinline__ void sfor_while(Fn&& f) {
 // The grouped projections run per unit: the pairs of one grouping tile (a
 // 64-pair half of a tile of more than kGroupWholeMax pairs, or a whole
 // smaller tile) times a block of 128 weight rows (gate/up: the gate and up rows
-// of 64 features; down: 128 outputs). Each of the four wavefronts owns RT = 2
-// 16-row A operands of v_mfma_f32_16x16x32_f16 and the whole K loop; the pairs
-// are NTT = 1, 2 or 4 16-pair B operands. Units of 256 rows (RT 4) spread an
+// of 64 features; down: 128 outputs, or 256 for small tiles where the host asks
+// for it). Each of the four wavefronts owns RT = 2 (4 for 256 rows) 16-row A
+// operands of v_mfma_f32_16x16x32_f16 and the whole K loop; the pairs are NTT = 1, 2 or 4 16-pair B operands. Units of 256 rows (RT 4) spread an
 // activation k-tile over twice the rows but are too few to share out evenly
 // over the blocks: 33 tokens of a 128-expert block are ~530 gate/up units of
 // them on 512 blocks, two rounds with the second nearly empty, and 704
-// features leave the last one half empty. With 128 rows: 512 tokens at 4 bits
+// features leave the last one half empty. Rows of few k-tiles are the exception
+// (the host's rule for down). With 128 rows: 512 tokens at 4 bits
 // 203.3 -> 195.5 us per call, 33 tokens at 3 bits 107.2 -> 104.6. Lane l holds
 // row l%16 of each A operand and the quarter q = l/16 of every 128-code k-tile
 // (chunk 4m + q: one 16-byte load at 4 bits;
@@ -507,15 +508,15 @@ __device__ __forceinline__ void unit_gate_up(const ExpertPool& pool, const Pair*
     }
 }
 
-// Down projection of one unit over 64·RT outputs of D (row block bx): wave
-// w takes rows d_blk + 16·RT·w + (0..16·RT-1). TAB as in unit_gate_up.
-template <int BITS, int NTT, bool TAB>
+// Down projection of one unit over 64·RT outputs of D (row block bx; RT 4 in
+// the launches of short rows): wave w takes rows d_blk + 16·RT·w +
+// (0..16·RT-1). TAB as in unit_gate_up.
+template <int BITS, int RT, int NTT, bool TAB>
 __device__ __forceinline__ void unit_down(const ExpertPool& pool, const Pair* __restrict__ sorted,
                                           const GroupedRows& gr, const uint16_t* __restrict__ act,
                                           uint16_t* __restrict__ partials, uint32_t D, uint32_t F, uint32_t k,
                                           uint32_t bx) {
     extern __shared__ __attribute__((aligned(16))) _Float16 unit_lds[];
-    constexpr int RT = kUnitRowTiles;
     constexpr uint32_t NR = 64u * RT;
     const uint32_t tid = unit_tid(), lane = tid & 63u, wave = tid >> 6;
     const uint32_t r16 = lane & 15u, q = lane >> 4;
@@ -545,8 +546,8 @@ __device__ __forceinline__ void unit_down(const ExpertPool& pool, const Pair* __
     const uint32_t nd = D - d_blk < NR ? D - d_blk : NR;
     const uint16_t* ds = reinterpret_cast<const uint16_t*>(blob + o.down_s) + (size_t)d_blk * G;
     const uint16_t* dbv = reinterpret_cast<const uint16_t*>(blob + o.down_b) + (size_t)d_blk * G;
-    TableRegs<1u> td;
-    unit_rows_loop<BITS, RT, NTT, kUnitDepth>(
+    TableRegs<TAB && RT == 4 ? 2u : 1u> td;
+    unit_rows_loop<BITS, RT, NTT, RT == 4 ? 4 : kUnitDepth>(
         wbase, woff, sbt, act, [&](uint32_t p) { return (gr.first + (p < gr.count ? p : 0u)) * F; }, F, unit_lds, acc,
         [&]() {
             if constexpr (TAB) td.issue(ds, dbv, nd * G, tid);
@@ -591,10 +592,10 @@ constexpr uint32_t kGroupNextUnit = 1, kGroupBlocksDone = 2;   // counter words 
 
 // Wavefront 0 writes the entries ({first pair, expert | count << 16}) of the
 // first min(n_tiles[0], max_tiles) tiles into ent; ends with a barrier and
-// returns how many there are.
-__device__ __forceinline__ uint32_t plan_units(const Tile* __restrict__ tiles, const uint32_t* __restrict__ n_tiles,
+// returns how many are half tiles (x, they come first) and how many there are (y).
+__device__ __forceinline__ uint2 plan_units(const Tile* __restrict__ tiles, const uint32_t* __restrict__ n_tiles,
                                                uint32_t max_tiles, uint2* ent) {
-    __shared__ uint32_t n_entries;
+    __shared__ uint2 n_entries;
     constexpr uint32_t C = kGroupMaxTiles / 64u;          // tiles per lane
     static_assert(kGroupMaxTiles % 64u == 0, "whole wavefront passes");
     if (threadIdx.x < 64u) {
@@ -654,29 +655,31 @@ __device__ __forceinline__ uint32_t plan_units(const Tile* __restrict__ tiles, c
                 ent[n0 + n1 + n2 + (pre_s[c] >> 16)] = make_uint2(t.start, t.expert | (t.count << 16));
             }
         }
-        if (lane == 0) n_entries = n0 + n1 + n2 + n3;
+        if (lane == 0) n_entries = make_uint2(n0 + n1, n0 + n1 + n2 + n3);
     }
     __syncthreads();
     return n_entries;
 }
 
-// The unit loop of one grouped launch: unit(rows, bx) runs one (block-uniform
-// calls). Every unit starts after a barrier, so it may reuse the dynamic LDS of
+// The unit loop of one grouped launch: unit(rows, bx, half tile or not) runs
+// one (block-uniform calls). Every unit starts after a barrier, so it may reuse the dynamic LDS of
 // the one before. state: the grouping state (tile count, then the counters).
 template <typename Unit>
 __device__ __forceinline__ void run_units(const Tile* __restrict__ tiles, uint32_t* __restrict__ state,
                                           GroupedLaunch gl, Unit unit) {
     __shared__ uint2 ent[kGroupMaxEntries];
     __shared__ uint32_t next_unit;
-    const uint32_t n_units = plan_units(tiles, state, gl.max_tiles, ent) * gl.row_blocks;
+    const uint2 n = plan_units(tiles, state, gl.max_tiles, ent);
+    const uint32_t n_half = n.x * gl.half_blocks, n_units = n_half + (n.y - n.x) * gl.small_blocks;
     const uint32_t P = gridDim.x, tid = threadIdx.x;
     uint32_t u = blockIdx.x;
     while (u < n_units) {
         // the next unit's number, asked for now and read after this unit
         uint32_t ask = 0;
         if (tid == 0) ask = atomicAdd(state + kGroupNextUnit, 1u);
-        const uint2 e = ent[u / gl.row_blocks];
-        unit(GroupedRows{e.x, e.y >> 16, e.y & 0xFFFFu}, u % gl.row_blocks);
+        const uint32_t v = u < n_half ? u : u - n_half, rb = u < n_half ? gl.half_blocks : gl.small_blocks;
+        const uint2 e = ent[(u < n_half ? 0u : n.x) + v / rb];
+        unit(GroupedRows{e.x, e.y >> 16, e.y & 0xFFFFu}, v % rb, u < n_half);
         if (tid == 0) next_unit = ask + P;
         __syncthreads();
         u = next_unit;
@@ -694,29 +697,34 @@ static_assert(kUnitThreads == kProjThreads, "the grouped launches run kProjThrea
 
 // TAB: the units' scale/bias tables staged through registers (the host
 // picks these launches for 16-byte aligned scale/bias offsets whose tables
-// fit: d <= 4096 for gate/up, f <= 1024 for down).
+// fit: d <= 4096 for gate/up, f <= 1024 for down). RS: RT of down's whole small
+// tiles.
 template <int BITS, bool TAB = false>
 __device__ __forceinline__ void moe_grouped_gate_up_launch(const ExpertPool& pool, const Pair* __restrict__ sorted,
                                                            const Tile* __restrict__ tiles, uint32_t* __restrict__ n_tiles,
                                                            const uint16_t* __restrict__ hidden, uint32_t stride,
                                                            uint16_t* __restrict__ act, uint32_t D, uint32_t F,
                                                            GroupedLaunch gl) {
-    run_units(tiles, n_tiles, gl, [&](const GroupedRows& gr, uint32_t bx) {
+    run_units(tiles, n_tiles, gl, [&](const GroupedRows& gr, uint32_t bx, bool) {
         if (gr.count <= 16u) unit_gate_up<BITS, 1, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
         else if (gr.count <= 32u) unit_gate_up<BITS, 2, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
         else unit_gate_up<BITS, 4, TAB>(pool, sorted, gr, hidden, stride, act, D, F, bx);
     });
 }
 
-template <int BITS, bool TAB = false>
+template <int BITS, int RS, bool TAB = false>
 __device__ __forceinline__ void moe_grouped_down_launch(const ExpertPool& pool, const Pair* __restrict__ sorted,
                                                         const Tile* __restrict__ tiles, uint32_t* __restrict__ n_tiles,
                                                         const uint16_t* __restrict__ act, uint16_t* __restrict__ partials,
                                                         uint32_t D, uint32_t F, uint32_t k, GroupedLaunch gl) {
-    run_units(tiles, n_tiles, gl, [&](const GroupedRows& gr, uint32_t bx) {
-        if (gr.count <= 16u) unit_down<BITS, 1, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
-        else if (gr.count <= 32u) unit_down<BITS, 2, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
-        else unit_down<BITS, 4, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
+    run_units(tiles, n_tiles, gl, [&](const GroupedRows& gr, uint32_t bx, bool half) {
+        if (half) {
+            if (gr.count <= 32u) unit_down<BITS, 2, 2, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
+            else unit_down<BITS, 2, 4, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
+        } else {
+            if (gr.count <= 16u) unit_down<BITS, RS, 1, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
+            else unit_down<BITS, RS, 2, TAB>(pool, sorted, gr, act, partials, D, F, k, bx);
+        }
     });
 }
 

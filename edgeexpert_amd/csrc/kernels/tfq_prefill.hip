@@ -9,8 +9,15 @@ extern "C" __global__ __launch_bounds__(kGroupThreads) void tfq_moe_group(
     moe_group(idx, w, T, k, E, sorted, offsets, counts, tiles, n_tiles, status);
 }
 
-// _t: the units' scale/bias tables staged through registers (aligned
-// tables that fit, chosen by the host)
+#define TFQ_GROUPED_DOWN(NAME, BITS, RS, TAB)                                                    \
+    extern "C" __global__ __launch_bounds__(kProjThreads, 2) void NAME(                           \
+        ExpertPool pool, const Pair* sorted, const Tile* tiles, uint32_t* n_tiles,               \
+        const uint16_t* act, uint16_t* partials, uint32_t D, uint32_t F, uint32_t k,             \
+        GroupedLaunch gl) {                                                                      \
+        moe_grouped_down_launch<BITS, RS, TAB>(pool, sorted, tiles, n_tiles, act, partials, D, F, k, gl); \
+    }
+// _t: the units' scale/bias tables staged through registers (aligned tables
+// that fit), _w: small tiles in units of 256 outputs (both chosen by the host)
 #define TFQ_GROUPED(SUFFIX, BITS, TAB)                                                           \
     extern "C" __global__ __launch_bounds__(kProjThreads, 2) void tfq_moe_grouped_gate_up##SUFFIX( \
         ExpertPool pool, const Pair* sorted, const Tile* tiles, uint32_t* n_tiles,               \
@@ -18,12 +25,8 @@ extern "C" __global__ __launch_bounds__(kGroupThreads) void tfq_moe_group(
         GroupedLaunch gl) {                                                                      \
         moe_grouped_gate_up_launch<BITS, TAB>(pool, sorted, tiles, n_tiles, hidden, stride, act, D, F, gl); \
     }                                                                                            \
-    extern "C" __global__ __launch_bounds__(kProjThreads, 2) void tfq_moe_grouped_down##SUFFIX(  \
-        ExpertPool pool, const Pair* sorted, const Tile* tiles, uint32_t* n_tiles,               \
-        const uint16_t* act, uint16_t* partials, uint32_t D, uint32_t F, uint32_t k,             \
-        GroupedLaunch gl) {                                                                      \
-        moe_grouped_down_launch<BITS, TAB>(pool, sorted, tiles, n_tiles, act, partials, D, F, k, gl); \
-    }
+    TFQ_GROUPED_DOWN(tfq_moe_grouped_down##SUFFIX, BITS, 2, TAB)                                  \
+    TFQ_GROUPED_DOWN(tfq_moe_grouped_down##SUFFIX##_w, BITS, 4, TAB)
 TFQ_GROUPED(, 4, false)
 TFQ_GROUPED(_b2, 2, false)
 TFQ_GROUPED(_b3, 3, false)

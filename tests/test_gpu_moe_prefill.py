@@ -417,6 +417,38 @@ def test_grouped_few_pairs_per_expert(ctx, stream, d, bits):
                         from_f16_bits(hidden).astype(np.float64).reshape(T, d), pool_bytes, offs, stride, d, f, k, bits)
 
 
+@pytest.mark.parametrize("bits,d,f,misaligned", [(4, 320, 64, False), (4, 320, 512, False), (4, 576, 320, True),
+                                                 (3, 320, 448, False), (2, 320, 704, False), (2, 512, 64, False)])
+def test_grouped_down_units_of_256_outputs(ctx, stream, bits, d, f, misaligned):
+    # short rows and enough tiles: down runs tiles of at most 32 pairs as units
+    # of 256 outputs beside the halves of larger ones: pair counts at both sides
+    # of the 16-pair sub-tiles and of the cut, partial row blocks (64
+    # outputs in the last), half-filled last k-tiles, tables through registers
+    # and copied
+    k, E = 1, 256
+    counts = [1, 15, 16, 17, 31, 32, 33, 0, 65, 129] + [0] * (E - 10)
+    T = sum(counts)
+    assert ops.max_tiles(T, k, E) * ((d + 255) // 256) >= 2 * 256
+    idx = np.repeat(np.arange(E, dtype=np.uint32), counts).reshape(T, k)
+    w16 = np.full((T, k), 0x3C00, np.uint16)
+    pool_bytes, offs, stride = synth.expert_pool(16, f"wide/{d}x{f}b{bits}", E, d, f, bits=bits)
+    dev, doffs, dstride = (_repack_misaligned(pool_bytes, offs, stride, E, d, f) if misaligned
+                           else (pool_bytes, offs, stride))
+    hidden = synth.f16_vector(16, "wide/x", T * d)
+    got, bufs = _device_group(ctx, stream, idx, w16, T, k, E)
+    pool = ops.ExpertPool(_dev(dev), dstride, E, doffs, weight_bits=bits)
+    act, partials = _dev(np.full(T * f, UNWRITTEN, np.uint16)), _dev(np.full(T * d, UNWRITTEN, np.uint16))
+    for _ in range(2):                    # the second call finds the counters zeroed
+        ops.PrefillGroupedRoutedMoE(ctx).encode(stream, pool, bufs["sorted"], bufs["tiles"], bufs["n_tiles"],
+                                                ops.max_tiles(T, k, E), _dev(hidden), d, d, f, k, act, partials)
+    stream.sync()
+    a, parts = act.download(np.uint16), partials.download(np.uint16)
+    assert not np.any(a == UNWRITTEN) and not np.any(parts == UNWRITTEN)
+    _check_grouped_fp16(from_f16_bits(a).astype(np.float64).reshape(T, f),
+                        from_f16_bits(parts).astype(np.float64).reshape(T, d), got["sorted"].astype(oracle.PAIR_DTYPE),
+                        from_f16_bits(hidden).astype(np.float64).reshape(T, d), pool_bytes, offs, stride, d, f, k, bits)
+
+
 def test_grouped_kernel_does_not_depend_on_the_tile_bound(ctx, stream):
     # full tiles with a launch bound that is the real tile count: no fewer
     # pairs for it, so the same kernels and bits as with the loose bound
