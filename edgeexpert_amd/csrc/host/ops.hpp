@@ -1075,12 +1075,19 @@ public:
         // have one or two: gate/up as a weight stream. Only where the caller
         // states the pairs: a tile bound says nothing of them (64 tiles may be
         // 64 pairs or 8192), and the stream reads a tile's weights again for
-        // every 16 of its pairs. Per call at 128 experts, top-8, 4 bits, with
-        // it and with the units: 2 tokens 42.7 and 49.1 us, 8 tokens 64.7 and
-        // 68.1, 12 tokens 73.9 and 74.4, 16 tokens 78.5 and 76.4
-        if (d <= 4096 && n_pairs && n_pairs <= pool.num_experts * 3u / 4u) {
+        // every 16 of its pairs. Its blocks (16 features of a tile) are many for
+        // wide experts, and beyond 3072 inputs only one fits a CU. us of gate/up
+        // and down with the units and with it, 128 experts, top-8, 4 bits: 2816 x
+        // 704, 2 tokens 36.7 and 31.0, 8 54.7 and 52.7, 12 61.6 and 61.2; 2816 x
+        // 1536, 2 tokens 51.7 and 47.8, 6 78.5 and 82.0, 12 100 and 114; 4096 x
+        // 704, 2 tokens 45.2 and 43.3, 3 51.1 and 53.9; 4096 x 1536, 1 token 46.8
+        // and 45.8, 8 114 and 160
+        const uint32_t cnt = (d + 1023) / 1024;
+        const uint64_t stream_blocks = (uint64_t)n_pairs * ((f + 15) / 16);
+        if (d <= 4096 && n_pairs && n_pairs <= pool.num_experts * 3u / 4u &&
+            stream_blocks <= (cnt == 4 ? 768u : 17000u / (cnt + 1))) {
             char name[48];
-            std::snprintf(name, sizeof(name), "tfq_moe_stream_gate_up_b%u_c%u", bits, (d + 1023) / 1024);
+            std::snprintf(name, sizeof(name), "tfq_moe_stream_gate_up_b%u_c%u", bits, cnt);
             void* a1[] = {&kp, &sorted, &tiles, &n_tiles, &hidden, &stride, &act, &d, &f};
             rc = launch2(m_, name, (f + 15) / 16, max_tiles, kSkinnyThreads, 0, stream, a1);
         } else {

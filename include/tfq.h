@@ -643,8 +643,8 @@ int tfq_moe_grouped(tfq_ctx *ctx, void *stream, const tfq_expert_pool *pool,
 
 /* tfq_moe_grouped for a caller that knows how many pairs were grouped
  * (n_pairs = T*top_k; 0: not known, the same as tfq_moe_grouped). At most 3/4
- * as many pairs as experts run gate/up as a weight stream (d <= 4096): the
- * same products, fp32 sums in another order, less time (2 tokens of top-8 over
+ * as many pairs as experts, and not too many for the width of the experts, run
+ * gate/up as a weight stream (d <= 4096): the same products, fp32 sums in another order, less time (2 tokens of top-8 over
  * 128 experts 42.7 instead of 49.1 us for the block). n_pairs chooses the
  * kernel only: a wrong count costs time, not results. */
 int tfq_moe_grouped_pairs(tfq_ctx *ctx, void *stream, const tfq_expert_pool *pool,

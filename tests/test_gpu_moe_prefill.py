@@ -472,6 +472,25 @@ def test_grouped_kernel_does_not_depend_on_the_tile_bound(ctx, stream):
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
 
 
+def test_grouped_wide_experts_keep_the_units(ctx, stream):
+    # few pairs, but more stream blocks than CUs hold: a stated pair count
+    # leaves the units' kernels, and so their bits
+    d, f, k, E, T = 4096, 2112, 2, 8, 3
+    idx = np.array([[0, 1], [2, 3], [0, 5]], np.uint32)
+    w16 = np.full((T, k), 0x3C00, np.uint16)
+    pool_bytes, offs, stride = synth.expert_pool(17, "wideexp", E, d, f)
+    pool, hidden = ops.ExpertPool(_dev(pool_bytes), stride, E, offs), _dev(synth.f16_vector(17, "wideexp/x", T * d))
+    got, bufs = _device_group(ctx, stream, idx, w16, T, k, E)
+    out = []
+    for pairs in (0, T * k):
+        act, partials = _dev(np.full(T * k * f, UNWRITTEN, np.uint16)), _dev(np.full(T * k * d, UNWRITTEN, np.uint16))
+        ops.PrefillGroupedRoutedMoE(ctx).encode(stream, pool, bufs["sorted"], bufs["tiles"], bufs["n_tiles"],
+                                                ops.max_tiles(T, k, E), hidden, d, d, f, k, act, partials, pairs=pairs)
+        stream.sync()
+        out.append((act.download(np.uint16), partials.download(np.uint16)))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+
+
 def _repack_misaligned(pool_bytes, offs, stride, E, d, f):
     # the same experts with every scale and bias array at a 2-byte (not
     # 16-byte) aligned offset, weight arrays still 16-byte aligned
