@@ -42,12 +42,13 @@ constexpr uint32_t q8_tile_lds_bytes(uint32_t k) {
     return 2u * (kQ8TileTok * 128u + kQ8TileRows * 64u) + 4u * kQ8TileRows * (k / 64u);
 }
 // router logits of a block of tokens on the matrix cores: from these many
-// tokens and (token, expert) pairs on. Its time hardly depends on the tokens
-// (128 experts x 2816: 8.8 us for 96 tokens, 9.3 for 512), the per-token form's
-// does (9.0 and 36.4; 40 experts x 1088: 5.4 against 10.8 us at 512 and 5.2
-// against 4.4 at 128).
+// tokens and (token, expert) pairs on. Its time hardly depends on the tokens,
+// the per-token form's does (with the selection, 128 experts x 2816: 12.2 us for
+// 96 tokens and 13.5 for 512 against 11.5 and 37.8, 128 tokens 12.2 against
+// 13.3; x 4096: 96 tokens 15.5 against 13.8, 128 15.7 against 17.7; x 1024: 96
+// tokens 8.0 against 8.8).
 constexpr uint32_t kRouterBlockTokens = 96;
-constexpr uint32_t kRouterBlockRows = 96 * 128;
+constexpr uint32_t router_block_rows(uint32_t d) { return (d > 2048 ? 112u : 96u) * 128u; }
 // the pipelined tile of the prefill GEMM (gemm.hpp proj_pl_lds_bytes)
 constexpr uint32_t proj_pl_lds_bytes(uint32_t k) { return 3u * kProjBM * 72u * 2u + 4u * kProjBN * (k / 64u); }
 static_assert(proj_pl_lds_bytes(kProjMaxK) <= 160u * 1024u, "pipelined tile exceeds the LDS of a CU");
@@ -957,7 +958,7 @@ public:
         char name[64];
         uint32_t E = r.num_experts;
         int rc;
-        if (T >= kRouterBlockTokens && (uint64_t)T * E >= kRouterBlockRows && aligned(hidden, 16) && stride % 8 == 0 &&
+        if (T >= kRouterBlockTokens && (uint64_t)T * E >= router_block_rows(d) && aligned(hidden, 16) && stride % 8 == 0 &&
             aligned(r.effective_scale, 16)) {
             // 16 tokens x 16 experts per block on the matrix cores (gemm_q8.hpp)
             std::snprintf(name, sizeof(name), "tfq_router_block_c%u", (d + 511) / 512);

@@ -58,7 +58,8 @@ def test_prefill_router_matches_per_token_reference(ctx, stream, T, E, D, k):
 
 @pytest.mark.parametrize("T,E,D,with_eff,scale", [
     (96, 128, 2816, True, 1.0), (97, 128, 64, False, 1.0), (130, 100, 704, True, 1e-4), (128, 256, 4096, True, 3e4),
-    (200, 65, 1088, False, 6e-6), (111, 112, 3648, True, 1.0)])
+    (200, 65, 1088, False, 6e-6), (111, 112, 3648, True, 1.0), (113, 128, 2816, True, 1.0),
+    (129, 112, 3648, True, 1.0)])
 def test_prefill_router_many_tokens(ctx, stream, T, E, D, with_eff, scale):
     # many tokens take the matrix-core form: partial expert and token tiles,
     # 1 .. 8 groups per wavefront (the last wavefronts with fewer or none),
@@ -85,6 +86,25 @@ def test_prefill_router_many_tokens(ctx, stream, T, E, D, with_eff, scale):
     # the selection is the per-token rule on these logits: value descending, index ascending
     order = np.stack([np.lexsort((np.arange(E), -row)) for row in got])[:, :k]
     assert np.array_equal(idx.download(np.uint32).reshape(T, k), order)
+
+
+@pytest.mark.parametrize("T,E,D", [(95, 256, 512), (95, 128, 2816), (96, 128, 2816), (111, 128, 4096)])
+def test_prefill_router_short_blocks_keep_the_token_form(ctx, stream, T, E, D):
+    # below the token and (token, expert) counts from which the matrix-core form
+    # is faster: the bits of the per-token form, which a hidden that is only
+    # 2-byte aligned takes
+    W, S, B = synth.int8_matrix(5, f"prs/{E}x{D}", E, D)
+    router = ops.Router(_dev(W), _dev(S), _dev(B), E, None, None)
+    H, k, out = synth.f16_vector(5, "prs/h", T * D), 8, []
+    for off in (0, 2):
+        hb = DeviceBuffer(T * D * 2 + 16)
+        hb.upload(H, offset=off)
+        idx, w16 = _dev(np.zeros(T * k, np.uint32)), _dev(np.zeros(T * k, np.uint16))
+        logits = _dev(np.zeros(T * E, np.float32))
+        ops.PrefillRouter(ctx).encode_gemma4_block(stream, router, hb.ptr(off), D, T, D, k, idx, w16, logits)
+        stream.sync()
+        out.append(logits.download(np.uint32))
+    assert np.array_equal(*out)
 
 
 def test_prefill_router_many_tokens_keeps_rows_apart(ctx, stream):
