@@ -27,7 +27,16 @@ constexpr uint32_t kUnitThreads = 256;          // grouped MoE units (moe_prefil
 constexpr uint32_t kUnitStride = 128 + 8;       // halves per LDS activation row of a unit
 constexpr uint32_t kGroupMaxTiles = 8192 / 128 + 256;  // tiles the device planner takes (moe_prefill.hpp)
 // int8 rows over a block of tokens (gemm_q8.hpp)
-constexpr uint32_t kQ8RowTokens = 4;            // most tokens that run the decode kernels once per token
+// Whether a block of tokens runs the decode kernels once per token: at most 4,
+// or so little work that the matrix cores' two launches, whose time is mostly
+// the length of their rows, take longer: ~0.45 us per million codes times
+// tokens against 0.5 us and 1.85 us per 1000 codes of both rows. us once per
+// token and on the matrix cores: 640 x 320, 5 tokens 5.8 and 7.9, 24 8.6 and 8.9,
+// 32 9.7 and 9.1; 1024 x 512, 8 tokens 7.2 and 9.2, 24 11.0 and 10.8; 2816 x 704, 5
+// tokens 10.7 and 12.6, 8 13.4 and 13.2; 2816 x 2112, 5 tokens 20.5 and 15.3.
+constexpr bool q8_once_per_token(uint64_t tokens, uint64_t d, uint64_t f) {
+    return tokens <= 4 || tokens * d * f <= 2000000u + 3900u * (d + f);
+}
 // most tokens on the K-split form. Both launches of a call, K-split and tile, at
 // 2816 x 2112: 48 tokens 27.1 and 35.8 us, 64: 30.6 and 36.0, 72: 36.0 and 35.5,
 // 96: 42.8 and 35.8; at 4096 x 4096 64 tokens 46.3 and 56.9, 65: 62.0 and 56.2.
@@ -655,12 +664,13 @@ private:
 // S/Kernels/MoE/SharedExpertInt8.swift:55-210: the fused int8 gate/up/act
 // (shared_int8_gate_up_act_simd; gate and up kept in fp32 up to the
 // activation) and the int8 down GEMV. tokens > 1 runs the same for a block
-// of inputs x + t·x_stride into y + t·y_stride, act_scratch [tokens][f]: up to
-// kQ8RowTokens tokens, and rows of x that are not 16-byte aligned, as the
-// decode kernels once per token (each row the decode form's bits), else on the
-// matrix cores (gemm_q8.hpp: the same factored fp32 sums in another order;
-// 13.7 against 53 us for 16 tokens at 2816 x 2112, 62 against 1463 for 512; at
-// 4 tokens 11.1 against 17.4, left to the rows for their bits).
+// of inputs x + t·x_stride into y + t·y_stride, act_scratch [tokens][f]: few
+// tokens or small matrices (q8_once_per_token), and rows of x that are not
+// 16-byte aligned, as the decode kernels once per token (each row the decode
+// form's bits), else on the matrix cores (gemm_q8.hpp: the same factored fp32
+// sums in another order; 13.7 against 53 us for 16 tokens at 2816 x 2112, 62
+// against 1463 for 512; at 4 tokens 11.1 against 17.4, left to the rows for
+// their bits).
 class SharedExpertInt8 {
 public:
     explicit SharedExpertInt8(const Module& m) : m_(m), gemv_(m) {}
@@ -685,7 +695,7 @@ public:
         Q8Mat u = {static_cast<const uint8_t*>(up.weights), up.scales, up.biases};
         NormArg na = stage;
         // a block of tokens on the matrix cores (gemm_q8.hpp)
-        if (tokens > kQ8RowTokens && na.mode == kStageCopy && aligned(x, 16) && x_stride % 8 == 0 &&
+        if (!q8_once_per_token(tokens, d, f) && na.mode == kStageCopy && aligned(x, 16) && x_stride % 8 == 0 &&
             aligned(act_scratch, 16)) {
             const Q8Mat dn = {static_cast<const uint8_t*>(down.weights), down.scales, down.biases};
             if (!aligned(dn.w, 16)) return fail(TFQ_E_INVAL, "weights are not 16-byte aligned");

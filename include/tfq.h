@@ -505,8 +505,8 @@ size_t tfq_prefill_shared_expert_workspace_bytes(uint32_t weight_bits, uint32_t 
 
 /* The shared expert over a block of `tokens` rows: y + t*y_stride =
  * shared(x + t*x_stride) for t < tokens (strides in halves). int8 weights
- * run up to 4 tokens (and rows of x that are not 16-byte aligned) on the
- * decode kernels, each row bit-identical to tfq_shared_expert_q8, and more
+ * run up to 4 tokens, blocks of little work (tokens*d*f up to 2e6 +
+ * 3900*(d + f)) and rows of x that are not 16-byte aligned on the decode kernels, each row bit-identical to tfq_shared_expert_q8, and more
  * tokens on the matrix cores with the same factored sums (exact products of
  * code and activation, fp32 accumulation, fp32 scale and bias) in another
  * order. int4 weights run the prefill GEMM:

@@ -167,9 +167,12 @@ def test_prefill_shared_expert_config4_shape(ctx, stream, bits, rows):
 
 
 @pytest.mark.parametrize("rows,d,f", [(5, 128, 64), (16, 192, 4096), (17, 4096, 320), (32, 2816, 704), (33, 64, 128),
-                                      (64, 320, 192), (65, 704, 2112), (130, 192, 64), (70, 64, 4096)])
+                                      (64, 320, 192), (65, 704, 2112), (130, 192, 64), (70, 64, 4096),
+                                      (6, 4096, 1088), (24, 192, 4096), (33, 1024, 320), (64, 320, 704),
+                                      (340, 128, 64), (400, 192, 64)])
 def test_prefill_shared_expert_int8_matrix_cores(ctx, stream, rows, d, f):
-    # from 5 tokens on the int8 block runs on the matrix cores: 16-token tiles
+    # more than 4 tokens of more than little work (the smallest sizes here stay
+    # once per token) run the int8 block on the matrix cores: 16-token tiles
     # with K split over eight wavefronts (up to 64 tokens; K from fewer groups
     # than wavefronts to 64), then 64 x 64 tiles (K of 1, 3, 5, 11, 33 and 64
     # groups); d and f leave partial row tiles, rows partial token tiles
@@ -182,11 +185,23 @@ def test_prefill_shared_expert_int8_matrix_cores(ctx, stream, rows, d, f):
         assert rel < TOL, f"row {r}: rel={rel}"
 
 
-@pytest.mark.parametrize("rows", [6, 66])
-def test_prefill_shared_expert_int8_keeps_rows_apart(ctx, stream, rows):
+@pytest.mark.parametrize("rows,d,f", [(5, 64, 64), (7, 2816, 704), (15, 1024, 512), (28, 640, 320), (130, 192, 64)])
+def test_prefill_shared_expert_int8_little_work_keeps_the_row_bits(ctx, stream, rows, d, f):
+    # blocks of little work: each row has the bits of the one-token form
+    mats = _synthetic(9, f"pshared8s/{d}x{f}", d, f, 8)
+    x, got = _prefill_case(ctx, stream, 8, rows, d, f, d + 8, d + 3, mats, 16)
+    for r in sorted({0, 1, rows // 2, rows - 1}):
+        y1 = _dev(np.zeros(d, np.uint16))
+        ops.SharedExpertInt8(ctx).encode(stream, _dev(x[r, :d]), _proj(mats[0], f, d), _proj(mats[1], f, d),
+                                         _proj(mats[2], d, f), y1, _dev(np.zeros(f, np.uint16)))
+        stream.sync()
+        assert np.array_equal(got[r].view(np.uint32), from_f16_bits(y1.download(np.uint16, d)).view(np.uint32)), f"row {r}"
+
+
+@pytest.mark.parametrize("rows,d,f", [(6, 256, 128), (66, 256, 128), (20, 1024, 512), (70, 1024, 512)])
+def test_prefill_shared_expert_int8_keeps_rows_apart(ctx, stream, rows, d, f):
     # an infinity in one row makes that row NaN (as inf * 0 codes and inf - inf
     # do in the decode form) and leaves every other row's bits as they were
-    d, f = 256, 128
     mats = _synthetic(8, "pshared8inf", d, f, 8)
     outs = []
     for bad in (False, True):
